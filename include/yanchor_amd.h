@@ -327,6 +327,37 @@ int yh_anchor_sequence_commit(const void* src_keys, const void* src_values, cons
                               int64_t chunk, int64_t D, int dtype, yh_stream_t stream);
 
 /*
+ * The three steps of a prefill that continues an anchor-memory state
+ * (yh_anchor_prefix, yh_anchor_sequence_read, yh_anchor_sequence_commit) with
+ * every row where it is: no assembled sources, no padded or reordered copies.
+ * New token i of row b is row (bases ? bases[b] : b * L) +
+ * (order ? order[b * L + i] : i) of the token tensors -- query [.., H, D], key /
+ * value [.., G, D] (token strides in elements), new_scores [.., G], out
+ * [.., H, D] -- so bases packs ragged rows and order (int32 [B, L], the valid
+ * tokens first) stands for a mask.  counts int64 [B]: valid new tokens; the
+ * tokens past counts[b] get zeros in out (with bases there are none).  keys .. total: the
+ * state, updated IN PLACE by the prefix (scores, positions, pending scores)
+ * and the commit (rows, count, total).  Otherwise as the calls above.
+ */
+int yh_anchor_tokens_prefix(const float* new_scores, const int64_t* bases, const int32_t* order,
+                            const int64_t* counts, float* scores, int32_t* positions, float* pending_scores,
+                            const int64_t* count, const int64_t* total, int32_t* block_refs, int32_t* final_refs,
+                            int32_t* pending_refs, int64_t B, int64_t L, int64_t G, int64_t capacity,
+                            int64_t pending_capacity, int64_t chunk, int64_t NB, yh_stream_t stream);
+int yh_anchor_tokens_read(const void* query, int64_t query_stride, const void* key, int64_t key_stride,
+                          const void* value, int64_t value_stride, const void* keys, const void* values,
+                          const void* pending_keys, const void* pending_values, const int32_t* references,
+                          const int64_t* first, const int64_t* counts, const int64_t* bases, const int32_t* order,
+                          void* out, int64_t B, int64_t L, int64_t NB, int64_t C, int64_t H, int64_t G, int64_t D,
+                          int64_t capacity, int64_t pending_capacity, int dtype, yh_stream_t stream);
+int yh_anchor_tokens_commit(const void* key, int64_t key_stride, const void* value, int64_t value_stride,
+                            const int32_t* final_refs, const int32_t* pending_refs, const int64_t* counts,
+                            const int64_t* bases, const int32_t* order, void* keys, void* values,
+                            void* pending_keys, void* pending_values, int64_t* count, int64_t* total, int64_t B,
+                            int64_t L, int64_t G, int64_t capacity, int64_t pending_capacity, int64_t chunk,
+                            int64_t D, int dtype, yh_stream_t stream);
+
+/*
  * Skinny bf16 projection of the decode step: out[M, N] = x[M, K] . W[N, K]^T,
  * fp32 accumulation, bf16 output (torch.nn.functional.linear without bias, the
  * q/k/v/z/b/a, output, MLP, memory-writer and lm_head projections of

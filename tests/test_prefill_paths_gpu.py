@@ -1,9 +1,13 @@
 """The prefill kernels at the sizes where their dispatch or tiling changes
 (GPU): runs, tiles and remainders, and rows that break 16-byte alignment."""
+from dataclasses import fields
+
 import pytest
 import torch
 
+from oracle import anchor as oracle_memory
 from oracle import glue
+from yanchor_amd import independent_memory as im
 from yanchor_amd import layers
 
 pytestmark = pytest.mark.gpu
@@ -86,3 +90,70 @@ def test_swa_prefill_tiles(gpu, heads, groups, window, lengths, starts, dtype):
     pick = torch.randperm(len(tiles), generator=gen)
     again = layers.swa_prefill(*args, gate=gate.to(gpu), tiles=tiles[pick])
     assert ((again.cpu().double() - ref).norm() / ref.norm()).item() < 2e-2
+
+
+def _memory_state(gen, b, g, cap, chunk, counts, base, dtype, odd):
+    """A memory state with committed slots in no particular order, ``counts``
+    pending tokens a row and positions below ``base``.  odd: tied scores, empty
+    slots with finite scores and slots at positions past the new tokens."""
+    st = im.IndependentMemoryState.empty(b, g, cap, chunk, 128, "cpu", dtype)
+    for x in (st.keys, st.values, st.pending_keys, st.pending_values):
+        x.copy_(torch.randn(x.shape, generator=gen))
+    pos = torch.stack([torch.randperm(base, generator=gen)[:cap] for _ in range(b * g)]).view(b, g, cap)
+    sc = torch.randn(b, g, cap, generator=gen)
+    if odd:
+        sc = sc.round()
+        pos = torch.where(torch.rand(pos.shape, generator=gen) < 0.2, -1, pos)
+        pos = torch.where(torch.rand(pos.shape, generator=gen) < 0.1, pos + 1000000, pos).clamp(min=-1)
+    st.positions.copy_(pos)
+    st.scores.copy_(sc)
+    st.pending_scores.copy_(torch.randn(st.pending_scores.shape, generator=gen))
+    st.count.copy_(torch.tensor(counts))
+    st.total.copy_(torch.tensor([base + c for c in counts]))
+    return st
+
+
+def _clone(st, dev):
+    return im.IndependentMemoryState(**{f.name: getattr(st, f.name).to(dev, copy=True) for f in fields(st)})
+
+
+@pytest.mark.parametrize("cap,chunk,length,heads,groups,odd", [
+    (16, 8, 40, 4, 2, True),           # many small blocks, ties
+    (256, 64, 100, 32, 8, False),      # less than two blocks
+    (256, 64, 4200, 4, 1, True),       # more tokens than one sort holds
+    (1030, 5, 3100, 3, 1, True),       # sizes off every power of two, a second sort of a few blocks
+    (3, 64, 1, 8, 8, False),           # one token, fewer slots than a run
+])
+def test_memory_sequence_segments(gpu, cap, chunk, length, heads, groups, odd):
+    """The state bit for bit against the oracle's token order, the read within
+    1e-2 of it; masked rows and packed rows alike."""
+    gen = torch.Generator().manual_seed(cap + length)
+    b, dt = 3, torch.bfloat16
+    st = _memory_state(gen, b, groups, cap, chunk, [0, chunk - 1, chunk // 2], max(2 * cap, 64), dt, odd)
+    q = torch.randn(b, length, heads, 128, generator=gen).to(dt)
+    k = torch.randn(b, length, groups, 128, generator=gen).to(dt)
+    v = torch.randn(b, length, 2 * groups, 128, generator=gen).to(dt)[:, :, groups:]      # a column view
+    sc = torch.randn(b, length, groups, generator=gen)
+    if odd:
+        sc = sc.round()
+    lens = [length, max(1, length // 3), max(1, length - 1)]
+    valid = torch.arange(length)[None] < torch.tensor(lens)[:, None]
+    if odd and length > 2:
+        valid[0, 1] = False                                                               # a hole
+    want_state = oracle_memory.MemoryState(**{f.name: getattr(st, f.name).clone() for f in fields(st)})
+    want = oracle_memory.sequence(q, k, v, sc, valid, chunk, want_state)
+    got_state = _clone(st, gpu)
+    got = im.sequence(q.to(gpu), k.to(gpu), v.to(gpu), sc.to(gpu), valid.to(gpu), chunk, got_state)
+    for f in fields(st):
+        a, w = getattr(got_state, f.name).cpu(), getattr(want_state, f.name)
+        assert torch.equal(a.double(), w.double()), f.name
+    assert (got.cpu().double() - want.double()).norm() <= 1e-2 * want.double().norm() + 1e-6
+    assert not got.cpu()[~valid].any()
+    # packed: the same tokens without padding
+    lens = valid.sum(1).tolist()
+    pack = [x.to(gpu)[valid.to(gpu)] for x in (q, k, v, sc)]
+    packed_state = _clone(st, gpu)
+    again = im.sequence_packed(*pack, _cu(lens, gpu), lens, chunk, packed_state)
+    for f in fields(st):
+        assert torch.equal(getattr(packed_state, f.name), getattr(got_state, f.name)), f.name
+    assert torch.equal(again, got[valid.to(gpu)])

@@ -45,6 +45,9 @@ SIGNATURES: dict[str, list] = {
     "yh_window_attend": [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i32, _p],
     "yh_anchor_commit": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64,
                          _i64, _i64, _i64, _p, _i64, _i64, _i32, _p],
+    "yh_anchor_tokens_prefix": [_p] * 12 + [_i64] * 7 + [_p],
+    "yh_anchor_tokens_read": [_p, _i64, _p, _i64, _p, _i64] + [_p] * 10 + [_i64] * 9 + [_i32, _p],
+    "yh_anchor_tokens_commit": [_p, _i64, _p, _i64] + [_p] * 11 + [_i64] * 7 + [_i32, _p],
     "yh_anchor_prefix": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _p],
     "yh_anchor_sequence_commit": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64,
                                   _i64, _i64, _i32, _p],

@@ -17,226 +17,149 @@
 // sink logit 0 with value 0).  As in the reference, P enters the PV product as
 // a hi + lo pair of 16-bit values, so the product keeps fp32 accuracy.
 //
-// Workgroup = 4 waves x 16 query rows; grid (B * NB * G, ceil(C * H/G / 64)).
-// Reference rows are gathered 64 at a time into LDS: K row-major (A operand
-// of S^T), V transposed (A operand of O^T).  The MFMA K-index order of the PV
-// product is permuted to match the lanes that hold each score, so P never
-// leaves registers.
-#include "common.h"
+// A workgroup of 4 waves takes 128 of a block's C * H/G query rows (attn_tile.h);
+// reference rows are gathered 64 at a time, straight into LDS.
+//
+// Source rows come in up to three parts (a state's committed slots, its
+// pending slots, the new tokens), so a prefill that continues a state reads
+// them where they are.
+#include "anchor_source.h"
+#include "attn_tile.h"
 
 namespace yh {
 namespace {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4v __attribute__((ext_vector_type(4)));
-
-constexpr int kD = 128;
-constexpr int kTile = 64;        // reference rows per LDS tile
-constexpr int kKPad = kD + 8;    // K row stride (elements): 272 B, conflict-free 16 B reads
-constexpr int kVPad = kTile + 4; // V^T row stride (elements): 136 B, conflict-free 8 B reads
+using attn::kD;
 
 struct IdxArgs {
   const uint16_t* q;
-  const uint16_t* k;
-  const uint16_t* v;
+  int64_t q_ts;
+  AnchorSource src;
   const void* refs;
-  uint16_t* out;
-  int NB, C, H, G, S, CAP, KB, ref64;
+  uint16_t* out;   // [.., H, D]
+  int64_t NB;
+  int C, H, G, CAP, ref64;
   float scale;
-  // tokens in place (yh_anchor_sequence_read): query / out [B, L, H, D]; the
-  // query at block position p = nb * C + t of row b is token p - first[b]
-  // (no token, no read, for p outside [first[b], first[b] + L))
+  // tokens in place (first != null): the query at block position
+  // p = nb * C + t of row b is token p - first[b] of the row (src.token_row);
+  // no token, no read, for p outside [first[b], first[b] + L); tokens past
+  // counts[b] read nothing and get zeros (packed rows have none)
   const int64_t* first;
-  int L;
+  const int64_t* counts;
 };
 
-template <int DT>
-struct Mfma;
-template <>
-struct Mfma<YH_BF16> {
-  typedef bf16x8_t vec;
-  static __device__ __forceinline__ f32x4v run(vec a, vec b, f32x4v c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint16_t round(float x) { return f32_to_bf16(x); }
-  static __device__ __forceinline__ float widen(uint16_t h) { return bf16_to_f32(h); }
-};
-template <>
-struct Mfma<YH_F16> {
-  typedef f16x8_t vec;
-  static __device__ __forceinline__ f32x4v run(vec a, vec b, f32x4v c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint16_t round(float x) { return f32_to_f16(x); }
-  static __device__ __forceinline__ float widen(uint16_t h) { return f16_to_f32(h); }
-};
+// Workgroup id: group fastest, then the row chunk, so the chunks of a block
+// gather their common rows through one XCD's L2 one after the other.
+template <int DT, int NW>
+__global__ void __launch_bounds__(NW * 64, 2) indexed_gqa_kernel(IdxArgs a) {
+  __shared__ attn::Rows stage[4];   // two buffers of key rows, two of value rows; then the output
+  attn::Rows *ktile = stage, *vtile = stage + 2;
 
-__device__ __forceinline__ uint32_t pack2(uint16_t lo, uint16_t hi) {
-  return static_cast<uint32_t>(lo) | (static_cast<uint32_t>(hi) << 16);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int R = a.H / a.G, rows = a.C * R, chunks = (rows + NW * attn::kRows - 1) / (NW * attn::kRows);
+  const int g = blockIdx.x % a.G;
+  const unsigned rest = blockIdx.x / a.G;
+  const int m0 = (rest % chunks) * NW * attn::kRows + w * attn::kRows;
+  const int64_t bb = rest / chunks;     // b * NB + block
+  const int64_t b = bb / a.NB, nb = bb - b * a.NB;
+
+  // query row m of the block -> its row of q / out, -1 for none; live: it reads
+  auto query_row = [&](int m, bool& live) -> int64_t {
+    live = m < rows;
+    if (!live) return -1;
+    const int t = m % a.C;
+    if (a.first == nullptr) return bb * a.C + t;
+    const int64_t i = nb * a.C + t - a.first[b];
+    live = i >= 0 && i < a.src.L;
+    if (!live) return -1;
+    if (a.counts != nullptr && i >= a.counts[b]) live = false;
+    if (!live && a.src.bases != nullptr) return -1;   // packed: the next row's tokens
+    return a.src.token_row(b, static_cast<int>(i));
+  };
+  const int m = m0 + (lane & 31);
+  bool live;
+  const int64_t qrow = query_row(m, live);
+
+  attn::State<DT> st;
+  st.init(true);
+  st.load_q(a.q + (live ? qrow * a.q_ts + (g * R + m / a.C) * kD : 0), live);
+  const bool wave_live = __any(live);
+
+  const int64_t ref_base = (bb * a.G + g) * a.CAP;
+  auto load_ref = [&](int start) -> int {   // this lane's reference of the tile, -1 for none
+    const int n = start + lane;
+    if (n >= a.CAP) return -1;
+    const int64_t r = a.ref64 ? static_cast<const int64_t*>(a.refs)[ref_base + n]
+                              : static_cast<const int32_t*>(a.refs)[ref_base + n];
+    return r >= 0 && r < a.src.S ? static_cast<int>(r) : -1;
+  };
+  auto gather = [&](int buf, int ref) {     // lane l's reference is row l of the tile
+    const uint16_t *kp = reinterpret_cast<const uint16_t*>(attn::zero_row), *vp = kp;
+    if (ref >= 0) {
+      kp = static_cast<const uint16_t*>(a.src.row(0, b, ref, g));
+      vp = static_cast<const uint16_t*>(a.src.row(1, b, ref, g));
+    }
+    const uint64_t ka = reinterpret_cast<uint64_t>(kp), va = reinterpret_cast<uint64_t>(vp);
+    attn::load_rows<NW>(ktile[buf], [&](int row, int e, const void* l) {
+      attn::copy16(reinterpret_cast<const uint16_t*>(__shfl(ka, row, 64)) + e, l);
+    });
+    attn::load_rows<NW>(vtile[buf], [&](int row, int e, const void* l) {
+      attn::copy16(reinterpret_cast<const uint16_t*>(__shfl(va, row, 64)) + e, l);
+    });
+  };
+  const float k2 = a.scale * 1.4426950408889634f;
+  int ref = load_ref(0);
+  uint64_t have = __ballot(ref >= 0), next = 0;
+  if (have) gather(0, ref);
+  ref = load_ref(attn::kTile);
+  int buf = 0;
+  for (int start = 0; start < a.CAP; start += attn::kTile, buf ^= 1) {
+    attn::copy_wait();
+    attn::tile_barrier();
+    next = __ballot(ref >= 0);   // the same in every wave
+    if (next) gather(buf ^ 1, ref);
+    ref = load_ref(start + 2 * attn::kTile);
+    if (have && wave_live) {
+      attn::f32x16 c[2];
+      st.scores(ktile[buf], c);
+      if (have != ~0ull)
+        st.mask(c, [&](int key, int half) { return (have >> (key + 4 * half)) & 1; });
+      st.template step<true>(c, vtile[buf], k2);
+    }
+    have = next;
+  }
+  attn::copy_wait();
+  attn::tile_barrier();
+
+  static_assert(NW * attn::kRows * 16 <= sizeof(stage) / 16, "output staging");
+  st.store(&stage[0][0] + w * attn::kRows * 16, [&](int row, int d0, uint4 o) {
+    bool lv;
+    const int64_t orow = query_row(m0 + row, lv);
+    if (orow < 0) return;
+    if (!lv) o = make_uint4(0, 0, 0, 0);
+    *reinterpret_cast<uint4*>(a.out + (orow * a.H + g * R + (m0 + row) / a.C) * kD + d0) = o;
+  });
 }
 
-template <int DT>
-__global__ void __launch_bounds__(256) indexed_gqa_kernel(IdxArgs a) {
-  using M = Mfma<DT>;
-  using vec = typename M::vec;
-  __shared__ __align__(16) uint16_t ks[kTile][kKPad];
-  __shared__ __align__(16) uint16_t vt[kD][kVPad];
-  __shared__ int rs[kTile];
-
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int R = a.H / a.G;
-  const int rows = a.C * R;
-  const int bg = blockIdx.x;
-  const int g = bg % a.G;
-  const int64_t bb = bg / a.G;          // b * NB + block
-  const int64_t b = bb / a.NB;
-  const int qn = lane & 15, quad = lane >> 4;
-  const int m = blockIdx.y * 64 + w * 16 + qn;  // query row of this lane (as the MFMA column)
-  bool mvalid = m < rows;
-  int64_t qrow;
-  if (a.first == nullptr) {
-    qrow = mvalid ? ((bb * a.C + m % a.C) * a.H + g * R + m / a.C) : 0;
-  } else {
-    const int64_t tok = (bb - b * a.NB) * a.C + m % a.C - a.first[b];
-    mvalid = mvalid && tok >= 0 && tok < a.L;
-    qrow = mvalid ? ((b * a.L + tok) * a.H + g * R + m / a.C) : 0;
-  }
-
-  // Q^T operand (B of S^T = K Q^T): lane holds Q[m][step*32 + quad*8 + 0..7].
-  vec qv[4];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    uint4 x = make_uint4(0, 0, 0, 0);
-    if (mvalid) x = *reinterpret_cast<const uint4*>(a.q + qrow * kD + s * 32 + quad * 8);
-    qv[s] = __builtin_bit_cast(vec, x);
-  }
-
-  f32x4v acc[kD / 16];
-#pragma unroll
-  for (int t = 0; t < kD / 16; ++t) acc[t] = f32x4v{0.f, 0.f, 0.f, 0.f};
-  float mx = 0.f, den = 1.f;  // the sink: logit 0, value 0
-
-  const int64_t kb = a.KB == 1 ? 0 : b;
-  const int64_t ref_base = static_cast<int64_t>(bg) * a.CAP;
-  for (int start = 0; start < a.CAP; start += kTile) {
-    __syncthreads();  // previous tile fully consumed
-    if (tid < kTile) {
-      const int n = start + tid;
-      int64_t r = -1;
-      if (n < a.CAP) {
-        r = a.ref64 ? static_cast<const int64_t*>(a.refs)[ref_base + n]
-                    : static_cast<const int32_t*>(a.refs)[ref_base + n];
-      }
-      rs[tid] = (r >= 0 && r < a.S) ? static_cast<int>(r) : -1;
-    }
-    __syncthreads();
-    const bool any = __syncthreads_or(tid < kTile && rs[tid] >= 0);
-    if (!any) continue;
-    // gather: 64 rows x 16 vectors of 8 elements, 4 vectors per thread
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const int idx = it * 256 + tid;
-      const int row = idx >> 4, c8 = (idx & 15) * 8;
-      const int r = rs[row];
-      uint4 kx = make_uint4(0, 0, 0, 0), vx = make_uint4(0, 0, 0, 0);
-      if (r >= 0) {
-        const int64_t off = ((kb * a.S + r) * a.G + g) * kD + c8;
-        kx = *reinterpret_cast<const uint4*>(a.k + off);
-        vx = *reinterpret_cast<const uint4*>(a.v + off);
-      }
-      *reinterpret_cast<uint4*>(&ks[row][c8]) = kx;
-      const uint16_t* vh = reinterpret_cast<const uint16_t*>(&vx);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) vt[c8 + j][row] = vh[j];
-    }
-    __syncthreads();
-
-    // S^T tiles: rt covers refs rt*16 .. +15; lane holds refs rt*16 + quad*4 + i
-    // for query column qn.
-    float sc[4][4];
-    float tmax = -INFINITY;
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      f32x4v c = f32x4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const vec kvv = __builtin_bit_cast(vec, *reinterpret_cast<const uint4*>(&ks[rt * 16 + qn][s * 32 + quad * 8]));
-        c = M::run(kvv, qv[s], c);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const bool live = rs[rt * 16 + quad * 4 + i] >= 0;
-        sc[rt][i] = live ? c[i] * a.scale : -INFINITY;
-        tmax = fmaxf(tmax, sc[rt][i]);
-      }
-    }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float nmx = fmaxf(mx, tmax);
-    const float alpha = __expf(mx - nmx);
-    float psum = 0.f;
-    uint16_t ph[4][4], pl[4][4];
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float p = __expf(sc[rt][i] - nmx);  // 0 for masked refs
-        psum += p;
-        ph[rt][i] = M::round(p);
-        pl[rt][i] = M::round(p - M::widen(ph[rt][i]));
-      }
-    }
-    psum += __shfl_xor(psum, 16, 64);
-    psum += __shfl_xor(psum, 32, 64);
-    den = den * alpha + psum;
-    mx = nmx;
-#pragma unroll
-    for (int t = 0; t < kD / 16; ++t) acc[t] *= alpha;
-
-    // O^T += V^T P^T over two 32-deep steps; K-index j of lane (quad) maps to
-    // ref 32s + quad*4 + j (j < 4) and 32s + 16 + quad*4 + j-4 (j >= 4).
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const vec phv = __builtin_bit_cast(
-          vec, make_uint4(pack2(ph[2 * s][0], ph[2 * s][1]), pack2(ph[2 * s][2], ph[2 * s][3]),
-                          pack2(ph[2 * s + 1][0], ph[2 * s + 1][1]), pack2(ph[2 * s + 1][2], ph[2 * s + 1][3])));
-      const vec plv = __builtin_bit_cast(
-          vec, make_uint4(pack2(pl[2 * s][0], pl[2 * s][1]), pack2(pl[2 * s][2], pl[2 * s][3]),
-                          pack2(pl[2 * s + 1][0], pl[2 * s + 1][1]), pack2(pl[2 * s + 1][2], pl[2 * s + 1][3])));
-#pragma unroll
-      for (int t = 0; t < kD / 16; ++t) {
-        const uint16_t* row = &vt[t * 16 + qn][0];
-        const uint2 lo = *reinterpret_cast<const uint2*>(row + 32 * s + quad * 4);
-        const uint2 hi = *reinterpret_cast<const uint2*>(row + 32 * s + 16 + quad * 4);
-        const vec vv = __builtin_bit_cast(vec, make_uint4(lo.x, lo.y, hi.x, hi.y));
-        acc[t] = M::run(vv, phv, acc[t]);
-        acc[t] = M::run(vv, plv, acc[t]);
-      }
-    }
-  }
-
-  if (!mvalid) return;
-  const float inv = 1.f / den;
-  uint16_t* orow = a.out + qrow * kD;
-#pragma unroll
-  for (int t = 0; t < kD / 16; ++t) {
-    const int d0 = t * 16 + quad * 4;
-    const uint2 o = make_uint2(pack2(M::round(acc[t][0] * inv), M::round(acc[t][1] * inv)),
-                               pack2(M::round(acc[t][2] * inv), M::round(acc[t][3] * inv)));
-    *reinterpret_cast<uint2*>(orow + d0) = o;
-  }
+int launch_indexed(IdxArgs a, int64_t B, int dtype, yh_stream_t stream, const char* what) {
+  constexpr int kWaves = 4;
+  const int64_t groups = B * a.NB * a.G;
+  const int64_t chunks = (static_cast<int64_t>(a.C) * (a.H / a.G) + kWaves * attn::kRows - 1) / (kWaves * attn::kRows);
+  YH_CHECK_ARG(groups < (1ll << 31) && groups * chunks < (1ll << 32) / (kWaves * 64), "%s: grid too large", what);
+  if (groups == 0) return YH_OK;
+  const dim3 grid(static_cast<unsigned>(groups * chunks)), block(kWaves * 64);
+  a.scale = 1.f / sqrtf(static_cast<float>(kD));
+  if (dtype == YH_BF16)
+    hipLaunchKernelGGL((indexed_gqa_kernel<YH_BF16, kWaves>), grid, block, 0, static_cast<hipStream_t>(stream), a);
+  else
+    hipLaunchKernelGGL((indexed_gqa_kernel<YH_F16, kWaves>), grid, block, 0, static_cast<hipStream_t>(stream), a);
+  YH_CHECK_LAUNCH(what);
+  return YH_OK;
 }
 
-}  // namespace
-}  // namespace yh
-
-namespace yh {
-namespace {
-int launch_indexed(const void* query, const void* key, const void* value, const void* references, int ref_dtype,
-                   void* out, int64_t B, int64_t NB, int64_t C, int64_t H, int64_t G, int64_t D, int64_t KB,
-                   int64_t S, int64_t CAP, const int64_t* first, int64_t L, int dtype, yh_stream_t stream,
-                   const char* what) {
+int check_indexed(const void* query, const void* key, const void* value, const void* references, int ref_dtype,
+                  const void* out, int64_t B, int64_t NB, int64_t C, int64_t H, int64_t G, int64_t D, int64_t KB,
+                  int64_t S, int64_t CAP, int64_t L, int dtype, const char* what) {
   YH_CHECK_ARG(B >= 0 && NB >= 0 && C > 0 && H > 0 && G > 0 && H % G == 0 && S >= 0 && CAP >= 0 && L >= 0,
                "%s: bad sizes", what);
   YH_CHECK_ARG(D == kD, "%s: head dim must be %d", what, kD);
@@ -246,33 +169,30 @@ int launch_indexed(const void* query, const void* key, const void* value, const 
     set_error("%s: dtype must be bf16 or fp16", what);
     return YH_ERR_UNSUPPORTED;
   }
-  const int64_t groups = B * NB * G;
-  if (groups == 0) return YH_OK;
+  if (B * NB * G == 0) return YH_OK;
   YH_CHECK_ARG(query && key && value && out && (CAP == 0 || references), "%s: null pointer", what);
   YH_CHECK_ARG(((reinterpret_cast<uintptr_t>(query) | reinterpret_cast<uintptr_t>(key) |
                  reinterpret_cast<uintptr_t>(value) | reinterpret_cast<uintptr_t>(out)) & 15) == 0,
                "%s: tensors must be 16-byte aligned", what);
-  YH_CHECK_ARG(groups < (1ll << 31) && C * (H / G) < (1ll << 20) && L < (1ll << 31), "%s: grid too large", what);
-  IdxArgs a{static_cast<const uint16_t*>(query), static_cast<const uint16_t*>(key),
-            static_cast<const uint16_t*>(value), references, static_cast<uint16_t*>(out), (int)NB, (int)C, (int)H,
-            (int)G, (int)S, (int)CAP, (int)KB, ref_dtype == YH_I64 ? 1 : 0, 1.f / sqrtf(static_cast<float>(D)),
-            first, (int)L};
-  const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>((C * (H / G) + 63) / 64));
-  if (dtype == YH_BF16)
-    hipLaunchKernelGGL(indexed_gqa_kernel<YH_BF16>, grid, dim3(256), 0, static_cast<hipStream_t>(stream), a);
-  else
-    hipLaunchKernelGGL(indexed_gqa_kernel<YH_F16>, grid, dim3(256), 0, static_cast<hipStream_t>(stream), a);
-  YH_CHECK_LAUNCH(what);
+  YH_CHECK_ARG(C * (H / G) < (1ll << 20) && L < (1ll << 31) && S < (1ll << 31) && CAP < (1ll << 30),
+               "%s: grid too large", what);
   return YH_OK;
 }
+
 }  // namespace
 }  // namespace yh
 
 extern "C" int yh_indexed_gqa(const void* query, const void* key, const void* value, const void* references,
                               int ref_dtype, void* out, int64_t B, int64_t NB, int64_t C, int64_t H, int64_t G,
                               int64_t D, int64_t KB, int64_t S, int64_t CAP, int dtype, yh_stream_t stream) {
-  return yh::launch_indexed(query, key, value, references, ref_dtype, out, B, NB, C, H, G, D, KB, S, CAP, nullptr, 0,
-                            dtype, stream, "indexed_gqa");
+  using namespace yh;
+  const int rc = check_indexed(query, key, value, references, ref_dtype, out, B, NB, C, H, G, D, KB, S, CAP, 0, dtype,
+                               "indexed_gqa");
+  if (rc != YH_OK || B * NB * G == 0) return rc;
+  IdxArgs a{static_cast<const uint16_t*>(query), H * D, assembled_source(key, value, KB == 1 ? 0 : S, S, G, D * 2),
+            references, static_cast<uint16_t*>(out), NB, (int)C, (int)H, (int)G, (int)CAP,
+            ref_dtype == YH_I64 ? 1 : 0, 0.f, nullptr, nullptr};
+  return launch_indexed(a, B, dtype, stream, "indexed_gqa");
 }
 
 extern "C" int yh_anchor_sequence_read(const void* query, const void* key, const void* value,
@@ -281,6 +201,39 @@ extern "C" int yh_anchor_sequence_read(const void* query, const void* key, const
                                        int64_t S, int64_t CAP, int dtype, yh_stream_t stream) {
   using namespace yh;
   YH_CHECK_ARG(first != nullptr || B == 0, "anchor_sequence_read: null pointer");
-  return launch_indexed(query, key, value, references, ref_dtype, out, B, NB, C, H, G, D, B, S, CAP, first, L, dtype,
-                        stream, "anchor_sequence_read");
+  const int rc = check_indexed(query, key, value, references, ref_dtype, out, B, NB, C, H, G, D, B, S, CAP, L, dtype,
+                               "anchor_sequence_read");
+  if (rc != YH_OK || B * NB * G == 0) return rc;
+  IdxArgs a{static_cast<const uint16_t*>(query), H * D, assembled_source(key, value, S, S, G, D * 2), references,
+            static_cast<uint16_t*>(out), NB, (int)C, (int)H, (int)G, (int)CAP, ref_dtype == YH_I64 ? 1 : 0, 0.f,
+            first, nullptr};
+  a.src.L = (int)L;        // query rows: token i of row b at b * L + i
+  a.src.batch_rows = L;
+  return launch_indexed(a, B, dtype, stream, "anchor_sequence_read");
+}
+
+extern "C" int yh_anchor_tokens_read(const void* query, int64_t query_stride, const void* key, int64_t key_stride,
+                                     const void* value, int64_t value_stride, const void* keys, const void* values,
+                                     const void* pending_keys, const void* pending_values, const int32_t* references,
+                                     const int64_t* first, const int64_t* counts, const int64_t* bases,
+                                     const int32_t* order, void* out, int64_t B, int64_t L, int64_t NB, int64_t C,
+                                     int64_t H, int64_t G, int64_t D, int64_t capacity, int64_t pending_capacity,
+                                     int dtype, yh_stream_t stream) {
+  using namespace yh;
+  const char* what = "anchor_tokens_read";
+  YH_CHECK_ARG(capacity > 0 && pending_capacity >= C, "%s: bad sizes", what);
+  const int rc = check_indexed(query, key, value, references, YH_I32, out, B, NB, C, H, G, D, B, capacity + C + L,
+                               capacity, L, dtype, what);
+  if (rc != YH_OK || B * NB * G == 0) return rc;
+  YH_CHECK_ARG(keys && values && pending_keys && pending_values && first && counts, "%s: null pointer", what);
+  YH_CHECK_ARG(((reinterpret_cast<uintptr_t>(keys) | reinterpret_cast<uintptr_t>(values) |
+                 reinterpret_cast<uintptr_t>(pending_keys) | reinterpret_cast<uintptr_t>(pending_values)) & 15) == 0 &&
+                   query_stride % 8 == 0 && key_stride % 8 == 0 && value_stride % 8 == 0 && query_stride >= H * D &&
+                   key_stride >= G * D && value_stride >= G * D,
+               "%s: rows must be 16-byte aligned and hold whole heads", what);
+  IdxArgs a{static_cast<const uint16_t*>(query), query_stride,
+            state_source(keys, values, pending_keys, pending_values, key, key_stride * 2, value, value_stride * 2, bases,
+                         order, L, C, G, capacity, pending_capacity, D * 2),
+            references, static_cast<uint16_t*>(out), NB, (int)C, (int)H, (int)G, (int)capacity, 0, 0.f, first, counts};
+  return launch_indexed(a, B, dtype, stream, what);
 }

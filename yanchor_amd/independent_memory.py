@@ -282,45 +282,79 @@ def sequence(query, key, value, scores, valid, chunk, state: IndependentMemorySt
         if not getattr(state, f.name).is_contiguous():
             raise ValueError(f"memory state field {f.name} must be contiguous")
     N.require_device(query, key, value, scores, valid, state.keys)
-    dev = query.device
-    bi = torch.arange(b, device=dev)[:, None]
     if valid is None:
         order = None
-        q, k, v, sc = query, key, value, scores
-        counts = torch.full((b,), length, device=dev, dtype=torch.long)
+        counts = torch.full((b,), length, device=query.device, dtype=torch.long)
     else:
-        order = valid.long().argsort(dim=1, descending=True, stable=True)
-        q, k, v, sc = (x[bi, order] for x in (query, key, value, scores))
-        counts = valid.sum(1)
+        order = valid.long().argsort(dim=1, descending=True, stable=True).to(torch.int32)
+        counts = valid.sum(1).to(torch.long)
+    out = torch.empty(query.shape, dtype=query.dtype, device=query.device)
+    _sequence_tokens(query.reshape(-1, h, d), key.reshape(-1, g, d), value.reshape(-1, g, d), scores, counts, None,
+                     order, length, c, state, out)
+    return out
+
+
+def sequence_packed(query, key, value, scores, cu_seqlens, lengths, chunk, state: IndependentMemoryState):
+    """``sequence`` over ragged rows packed without padding: row r holds
+    tokens [cu_seqlens[r], cu_seqlens[r + 1]) of query ``[N, H, D]``, key /
+    value ``[N, G, D]`` and scores ``[N, G]`` (``lengths``: the same lengths on
+    the host, each >= 1).  Returns the read ``[N, H, D]``."""
+    nb, g, cap, pc, d = _check_state(state)
+    n, h = query.shape[:2]
+    if query.shape != (n, h, d) or key.shape != (n, g, d) or value.shape != key.shape or scores.shape != (n, g):
+        raise ValueError("query must be [N, H, D], key/value [N, G, D] and scores [N, G] matching the memory")
+    if nb != len(lengths) or cu_seqlens.shape != (nb + 1,) or sum(lengths) != n or min(lengths) < 1:
+        raise ValueError("the memory state must have one row per packed row of at least one token")
+    c = int(chunk)
+    if not 1 <= c <= pc:
+        raise ValueError(f"chunk {chunk} must lie in [1, {pc}]")
+    if query.dtype != state.keys.dtype or key.dtype != state.keys.dtype or value.dtype != state.keys.dtype:
+        raise ValueError("query/key/value must match the memory dtype")
+    for f in fields(state):
+        if not getattr(state, f.name).is_contiguous():
+            raise ValueError(f"memory state field {f.name} must be contiguous")
+    N.require_device(query, key, value, scores, cu_seqlens, state.keys)
+    cu = cu_seqlens.to(torch.long)
+    out = torch.empty(query.shape, dtype=query.dtype, device=query.device)
+    _sequence_tokens(query, key, value, scores, cu[1:] - cu[:-1], cu, None, max(lengths), c, state, out)
+    return out
+
+
+def _token_rows(x):
+    """x [N, heads, D] with heads contiguous and 16-byte aligned rows (any
+    token stride, in order), copied where it is not."""
+    if x.stride(2) == 1 and x.stride(1) == x.shape[2] and x.stride(0) >= x.shape[1] * x.shape[2] and \
+            x.stride(0) * x.element_size() % 16 == 0 and x.data_ptr() % 16 == 0:
+        return x
+    return x.clone(memory_format=torch.contiguous_format)
+
+
+def _sequence_tokens(query, key, value, scores, counts, bases, order, length, c, state, out):
+    """The prefix Top-K scan, the read and the state rewrite on tokens in
+    place (yh_anchor_tokens_*): query [N, H, D], key / value [N, G, D]."""
+    b, g, cap, d = state.keys.shape
+    pc, h, dev = state.pending_keys.shape[2], query.shape[1], query.device
     blocks = -(-length // c) + 1                  # ceil((L + C) / C) blocks of C positions
-    src_k = torch.cat((state.keys.transpose(1, 2), state.pending_keys[:, :, :c].transpose(1, 2), k), 1).contiguous()
-    src_v = torch.cat((state.values.transpose(1, 2), state.pending_values[:, :, :c].transpose(1, 2), v),
-                      1).contiguous()
-    n_src = cap + c + length
     block_refs = torch.empty(b, blocks, g, cap, device=dev, dtype=torch.int32)
     final_refs = torch.empty(b, g, cap, device=dev, dtype=torch.int32)
     pending_refs = torch.empty(b, g, pc, device=dev, dtype=torch.int32)
-    sc = sc.to(torch.float32).contiguous()
-    counts = counts.to(torch.long).contiguous()
+    sc = scores.to(torch.float32).contiguous()
+    q, k, v = (_token_rows(x) for x in (query, key, value))
     st = N.stream_of(query)
-    N.call("yh_anchor_prefix", sc.data_ptr(), counts.data_ptr(), state.scores.data_ptr(),
-           state.positions.data_ptr(), state.pending_scores.data_ptr(), state.count.data_ptr(),
-           state.total.data_ptr(), block_refs.data_ptr(), final_refs.data_ptr(), pending_refs.data_ptr(), b, length,
-           g, cap, pc, c, blocks, st)
-    # block position p of row b reads token p - old[b] in place (the old
+    N.call("yh_anchor_tokens_prefix", sc.data_ptr(), N.ptr(bases), N.ptr(order), counts.data_ptr(),
+           state.scores.data_ptr(), state.positions.data_ptr(), state.pending_scores.data_ptr(),
+           state.count.data_ptr(), state.total.data_ptr(), block_refs.data_ptr(), final_refs.data_ptr(),
+           pending_refs.data_ptr(), b, length, g, cap, pc, c, blocks, st)
+    # block position p of row b reads token p - count[b] in place (the old
     # pending tokens open the first block and read nothing here)
-    first = state.count.contiguous()
-    qc = q.contiguous()
-    out = torch.empty_like(qc)
-    N.call("yh_anchor_sequence_read", qc.data_ptr(), src_k.data_ptr(), src_v.data_ptr(), block_refs.data_ptr(),
-           N.I32, first.data_ptr(), out.data_ptr(), b, length, blocks, c, h, g, d, n_src, cap, N.code(qc), st)
-    if order is not None:
-        out = out[bi, order.argsort(1)] * valid[..., None, None].to(out.dtype)
-    N.call("yh_anchor_sequence_commit", src_k.data_ptr(), src_v.data_ptr(), final_refs.data_ptr(),
-           pending_refs.data_ptr(), counts.data_ptr(), state.keys.data_ptr(), state.values.data_ptr(),
-           state.pending_keys.data_ptr(), state.pending_values.data_ptr(), state.count.data_ptr(),
-           state.total.data_ptr(), b, n_src, length, g, cap, pc, c, d, N.code(src_k), st)
-    return out
+    N.call("yh_anchor_tokens_read", q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
+           state.keys.data_ptr(), state.values.data_ptr(), state.pending_keys.data_ptr(),
+           state.pending_values.data_ptr(), block_refs.data_ptr(), state.count.data_ptr(), counts.data_ptr(),
+           N.ptr(bases), N.ptr(order), out.data_ptr(), b, length, blocks, c, h, g, d, cap, pc, N.code(q), st)
+    N.call("yh_anchor_tokens_commit", k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), final_refs.data_ptr(),
+           pending_refs.data_ptr(), counts.data_ptr(), N.ptr(bases), N.ptr(order), state.keys.data_ptr(),
+           state.values.data_ptr(), state.pending_keys.data_ptr(), state.pending_values.data_ptr(),
+           state.count.data_ptr(), state.total.data_ptr(), b, length, g, cap, pc, c, d, N.code(k), st)
 
 
 def ring_decode_attention(query, keys, values, positions, indices=None, gate=None):

@@ -284,6 +284,10 @@ class HipOps:
             return self.mem.sequence(q, key, value, scores, valid, chunk, state)
         return _token_by_token_sequence(self, q, key, value, scores, valid, chunk, state)
 
+    def memory_sequence_packed(self, q, key, value, scores, cu, lens, chunk, state):
+        """The same over packed rows of the given lengths (>= 1), 16-bit."""
+        return self.mem.sequence_packed(q, key, value, scores, cu, lens, chunk, state)
+
     def sample(self, logits, attempt_ids, steps, seen, *, seed, temperature, top_k, top_p, penalty,
                backend="triton_top20"):
         """One token per row with the presence penalty of ``seen`` fused in:
@@ -925,15 +929,18 @@ class Model:
         out = F.linear(att.reshape(n, H * D), L["w_o"])
         u = ops.rmsnorm(hidden, L["m_in_norm"], c.rms_eps)
         mq, mgate, mk, mv, msc = self._memory_decode(L, hidden, cos, sin, u)
-        read = self._memory_prefill(tmp.memory[i], mq, mk, mv, msc, lens)
+        read = self._memory_prefill(tmp.memory[i], mq, mk, mv, msc, lens, cu)
         return out + F.linear((read * mgate[..., None].to(read.dtype)).reshape(n, H * D), L["m_o"])
 
-    def _memory_prefill(self, state, q, key, value, scores, lens):
-        """_sequence over packed pieces: the rows with tokens are laid out as
-        a right-padded [R', Lmax] batch (padding invalid, which _sequence's
-        stable argsort takes as absent) on their own state rows; returns the
-        read of every packed token [N, H, D]."""
+    def _memory_prefill(self, state, q, key, value, scores, lens, cu):
+        """_sequence over packed pieces; returns the read of every packed
+        token [N, H, D].  Where every row has tokens the kernels take the
+        packed rows as they are; else the rows with tokens are laid out as a
+        right-padded [R', Lmax] batch (padding invalid, which _sequence's
+        stable argsort takes as absent) on their own state rows."""
         c, dev = self.cfg, q.device
+        if min(lens) and q.dtype in (torch.bfloat16, torch.float16) and hasattr(self.ops, "memory_sequence_packed"):
+            return self.ops.memory_sequence_packed(q, key, value, scores, cu, lens, c.memory_chunk, state)
         live = [r for r, n in enumerate(lens) if n]
         nl = [lens[r] for r in live]
         lmax = max(nl)
