@@ -39,6 +39,7 @@ struct IdxArgs {
   uint16_t* out;   // [.., H, D]
   int64_t NB;
   int C, H, G, CAP, ref64;
+  int per;         // blocks a workgroup walks
   float scale;
   // tokens in place (first != null): the query at block position
   // p = nb * C + t of row b is token p - first[b] of the row (src.token_row);
@@ -48,49 +49,72 @@ struct IdxArgs {
   const int64_t* counts;
 };
 
+// A workgroup walks `per` consecutive blocks of one (row, group) and one chunk
+// of their query rows: a block has only a few tiles, so the first gather and
+// the queries of the next block are in flight while the last tile of this one
+// is computed (one block a workgroup left the chip waiting for both; the whole
+// call at 32 rows of 2048 tokens, 256 slots: 794 us then, 743 us so).
+//
 // Workgroup id: group fastest, then the row chunk, so the chunks of a block
 // gather their common rows through one XCD's L2 one after the other.
 template <int DT, int NW>
 __global__ void __launch_bounds__(NW * 64, 2) indexed_gqa_kernel(IdxArgs a) {
-  __shared__ attn::Rows stage[4];   // two buffers of key rows, two of value rows; then the output
-  attn::Rows *ktile = stage, *vtile = stage + 2;
+  static_assert(NW == 4, "the output stages in the 32 KB of one tile");
+  __shared__ attn::Rows ktile[2], vtile[2];
 
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int R = a.H / a.G, rows = a.C * R, chunks = (rows + NW * attn::kRows - 1) / (NW * attn::kRows);
   const int g = blockIdx.x % a.G;
-  const unsigned rest = blockIdx.x / a.G;
+  unsigned rest = blockIdx.x / a.G;
   const int m0 = (rest % chunks) * NW * attn::kRows + w * attn::kRows;
-  const int64_t bb = rest / chunks;     // b * NB + block
-  const int64_t b = bb / a.NB, nb = bb - b * a.NB;
+  rest /= chunks;
+  const unsigned segs = static_cast<unsigned>((a.NB + a.per - 1) / a.per);
+  const int64_t b = rest / segs;
+  int64_t nb = static_cast<int64_t>(rest % segs) * a.per;
+  const int blocks = static_cast<int>(min(a.NB - nb, static_cast<int64_t>(a.per)));
 
-  // query row m of the block -> its row of q / out, -1 for none; live: it reads
-  auto query_row = [&](int m, bool& live) -> int64_t {
+  // query row m of block n -> its row of q / out, -1 for none; live: it reads
+  auto query_row = [&](int64_t n, int m, bool& live) -> int64_t {
+    asm volatile("" : "+v"(m));   // its quotients are formed where used, not kept over the blocks in registers
     live = m < rows;
     if (!live) return -1;
-    const int t = m % a.C;
-    if (a.first == nullptr) return bb * a.C + t;
-    const int64_t i = nb * a.C + t - a.first[b];
+    const int t = static_cast<unsigned>(m) % static_cast<unsigned>(a.C);
+    if (a.first == nullptr) return (b * a.NB + n) * a.C + t;
+    const int64_t i = n * a.C + t - a.first[b];
     live = i >= 0 && i < a.src.L;
     if (!live) return -1;
     if (a.counts != nullptr && i >= a.counts[b]) live = false;
     if (!live && a.src.bases != nullptr) return -1;   // packed: the next row's tokens
     return a.src.token_row(b, static_cast<int>(i));
   };
-  const int m = m0 + (lane & 31);
-  bool live;
-  const int64_t qrow = query_row(m, live);
+  attn::State<DT, true> st;
+  auto load_queries = [&](int64_t n) -> bool {   // whether any query of the wave reads
+    int m = m0 + (lane & 31);
+    asm volatile("" : "+v"(m));
+    bool live;
+    const int64_t qrow = query_row(n, m, live);
+    st.load_q(a.q + (live ? qrow * a.q_ts + (g * R + static_cast<unsigned>(m) / static_cast<unsigned>(a.C)) * kD : 0),
+              live);
+    return __any(live);
+  };
 
-  attn::State<DT> st;
-  st.init(true);
-  st.load_q(a.q + (live ? qrow * a.q_ts + (g * R + m / a.C) * kD : 0), live);
-  const bool wave_live = __any(live);
-
-  const int64_t ref_base = (bb * a.G + g) * a.CAP;
-  auto load_ref = [&](int start) -> int {   // this lane's reference of the tile, -1 for none
-    const int n = start + lane;
-    if (n >= a.CAP) return -1;
-    const int64_t r = a.ref64 ? static_cast<const int64_t*>(a.refs)[ref_base + n]
-                              : static_cast<const int32_t*>(a.refs)[ref_base + n];
+  const int tiles = max(1, (a.CAP + attn::kTile - 1) / attn::kTile);   // of a block
+  const int64_t ref_base = (b * a.NB * a.G + g) * a.CAP, ref_block = static_cast<int64_t>(a.G) * a.CAP;
+  // this lane's reference of a tile, -1 for none; the tiles one after the other
+  int64_t ref_nb = nb;
+  int ref_left = blocks, ref_start = 0;
+  auto next_ref = [&]() -> int {
+    int64_t r = -1;
+    if (ref_left > 0 && ref_start + lane < a.CAP) {
+      const int64_t at = ref_base + ref_nb * ref_block + ref_start + lane;
+      r = a.ref64 ? static_cast<const int64_t*>(a.refs)[at] : static_cast<const int32_t*>(a.refs)[at];
+    }
+    ref_start += attn::kTile;
+    if (ref_start >= a.CAP) {
+      ref_start = 0;
+      ++ref_nb;
+      --ref_left;
+    }
     return r >= 0 && r < a.src.S ? static_cast<int>(r) : -1;
   };
   auto gather = [&](int buf, int ref) {     // lane l's reference is row l of the tile
@@ -108,46 +132,64 @@ __global__ void __launch_bounds__(NW * 64, 2) indexed_gqa_kernel(IdxArgs a) {
     });
   };
   const float k2 = a.scale * 1.4426950408889634f;
-  int ref = load_ref(0);
+  int ref = next_ref();
+  st.init(true);
+  bool wave_live = load_queries(nb);
   uint64_t have = __ballot(ref >= 0), next = 0;
   if (have) gather(0, ref);
-  ref = load_ref(attn::kTile);
-  int buf = 0;
-  for (int start = 0; start < a.CAP; start += attn::kTile, buf ^= 1) {
+  ref = next_ref();
+  int buf = 0, tile = 0;
+  for (int left = blocks; left > 0; buf ^= 1) {
     attn::copy_wait();
     attn::tile_barrier();
     next = __ballot(ref >= 0);   // the same in every wave
     if (next) gather(buf ^ 1, ref);
-    ref = load_ref(start + 2 * attn::kTile);
+    ref = next_ref();
+    const bool last = ++tile == tiles;
+    bool live_after = false;
     if (have && wave_live) {
       attn::f32x16 c[2];
       st.scores(ktile[buf], c);
+      if (last && left > 1) live_after = load_queries(nb + 1);   // the scores are the last use of this block's
       if (have != ~0ull)
         st.mask(c, [&](int key, int half) { return (have >> (key + 4 * half)) & 1; });
       st.template step<true>(c, vtile[buf], k2);
+    } else if (last && left > 1) {
+      live_after = load_queries(nb + 1);
     }
     have = next;
+    if (!last) continue;
+    attn::tile_barrier();   // the tile is consumed: its LDS stages the output
+    st.store((w < 2 ? &ktile[buf][0] : &vtile[buf][0]) + (w & 1) * attn::kRows * 16, [&](int row, int d0, uint4 o) {
+      bool lv;
+      int m = m0 + row;
+      asm volatile("" : "+v"(m));
+      const int64_t orow = query_row(nb, m, lv);
+      if (orow < 0) return;
+      if (!lv) o = make_uint4(0, 0, 0, 0);
+      *reinterpret_cast<uint4*>(a.out + (orow * a.H + g * R + static_cast<unsigned>(m) / static_cast<unsigned>(a.C)) * kD + d0) = o;
+    });
+    st.init(true);
+    wave_live = live_after;
+    tile = 0;
+    ++nb;
+    --left;
   }
   attn::copy_wait();
-  attn::tile_barrier();
-
-  static_assert(NW * attn::kRows * 16 <= sizeof(stage) / 16, "output staging");
-  st.store(&stage[0][0] + w * attn::kRows * 16, [&](int row, int d0, uint4 o) {
-    bool lv;
-    const int64_t orow = query_row(m0 + row, lv);
-    if (orow < 0) return;
-    if (!lv) o = make_uint4(0, 0, 0, 0);
-    *reinterpret_cast<uint4*>(a.out + (orow * a.H + g * R + (m0 + row) / a.C) * kD + d0) = o;
-  });
 }
 
 int launch_indexed(IdxArgs a, int64_t B, int dtype, yh_stream_t stream, const char* what) {
   constexpr int kWaves = 4;
   const int64_t groups = B * a.NB * a.G;
-  const int64_t chunks = (static_cast<int64_t>(a.C) * (a.H / a.G) + kWaves * attn::kRows - 1) / (kWaves * attn::kRows);
-  YH_CHECK_ARG(groups < (1ll << 31) && groups * chunks < (1ll << 32) / (kWaves * 64), "%s: grid too large", what);
   if (groups == 0) return YH_OK;
-  const dim3 grid(static_cast<unsigned>(groups * chunks)), block(kWaves * 64);
+  const int64_t chunks = (static_cast<int64_t>(a.C) * (a.H / a.G) + kWaves * attn::kRows - 1) / (kWaves * attn::kRows);
+  // blocks a workgroup: as many as leave four workgroups for each of the 512
+  // that the chip holds
+  const int64_t per = groups * chunks / 2048;
+  a.per = static_cast<int>(per < 1 ? 1 : per > 8 ? 8 : per);
+  const int64_t wgs = B * ((a.NB + a.per - 1) / a.per) * a.G * chunks;
+  YH_CHECK_ARG(groups < (1ll << 31) && wgs < (1ll << 32) / (kWaves * 64), "%s: grid too large", what);
+  const dim3 grid(static_cast<unsigned>(wgs)), block(kWaves * 64);
   a.scale = 1.f / sqrtf(static_cast<float>(kD));
   if (dtype == YH_BF16)
     hipLaunchKernelGGL((indexed_gqa_kernel<YH_BF16, kWaves>), grid, block, 0, static_cast<hipStream_t>(stream), a);
@@ -191,7 +233,7 @@ extern "C" int yh_indexed_gqa(const void* query, const void* key, const void* va
   if (rc != YH_OK || B * NB * G == 0) return rc;
   IdxArgs a{static_cast<const uint16_t*>(query), H * D, assembled_source(key, value, KB == 1 ? 0 : S, S, G, D * 2),
             references, static_cast<uint16_t*>(out), NB, (int)C, (int)H, (int)G, (int)CAP,
-            ref_dtype == YH_I64 ? 1 : 0, 0.f, nullptr, nullptr};
+            ref_dtype == YH_I64 ? 1 : 0, 1, 0.f, nullptr, nullptr};
   return launch_indexed(a, B, dtype, stream, "indexed_gqa");
 }
 
@@ -205,7 +247,7 @@ extern "C" int yh_anchor_sequence_read(const void* query, const void* key, const
                                "anchor_sequence_read");
   if (rc != YH_OK || B * NB * G == 0) return rc;
   IdxArgs a{static_cast<const uint16_t*>(query), H * D, assembled_source(key, value, S, S, G, D * 2), references,
-            static_cast<uint16_t*>(out), NB, (int)C, (int)H, (int)G, (int)CAP, ref_dtype == YH_I64 ? 1 : 0, 0.f,
+            static_cast<uint16_t*>(out), NB, (int)C, (int)H, (int)G, (int)CAP, ref_dtype == YH_I64 ? 1 : 0, 1, 0.f,
             first, nullptr};
   a.src.L = (int)L;        // query rows: token i of row b at b * L + i
   a.src.batch_rows = L;
@@ -234,6 +276,6 @@ extern "C" int yh_anchor_tokens_read(const void* query, int64_t query_stride, co
   IdxArgs a{static_cast<const uint16_t*>(query), query_stride,
             state_source(keys, values, pending_keys, pending_values, key, key_stride * 2, value, value_stride * 2, bases,
                          order, L, C, G, capacity, pending_capacity, D * 2),
-            references, static_cast<uint16_t*>(out), NB, (int)C, (int)H, (int)G, (int)capacity, 0, 0.f, first, counts};
+            references, static_cast<uint16_t*>(out), NB, (int)C, (int)H, (int)G, (int)capacity, 0, 1, 0.f, first, counts};
   return launch_indexed(a, B, dtype, stream, what);
 }

@@ -18,8 +18,9 @@
 // and on the tile's barrier.  Hence: key tiles by direct global-to-LDS copies,
 // double buffered, one barrier a tile; 16-byte pieces swizzled so that the
 // 16-byte K reads and the transposing V reads hit distinct banks; a few
-// operands read ahead of their MFMA; a raised wave priority around the MFMAs,
-// so that one wave's MFMAs run under the other's vector work; no mask code on
+// operands read ahead of their MFMA; the exponentials of one step of the value
+// product between the MFMAs of the step before; a raised wave priority around
+// the MFMAs, so that they run under the other wave's vector work; no mask code on
 // tiles where every key is live.  Six waves a workgroup (three a SIMD, 168
 // registers) spill and take 1.7 times as long.  The denominator sums the
 // rounded P that the value product sees (two at a time, v_dot2), so the
@@ -128,8 +129,16 @@ __device__ __forceinline__ void load_rows(Rows& t, CopyFn copy) {
   }
 }
 
-template <int DT>
+// FRESH: LDS addresses are formed in every tile instead of staying in registers
+// over the tile loop, where a kernel's own invariants leave no room for them (a
+// spilled one is reloaded behind the copies in flight).
+template <int DT, bool FRESH = false>
 struct State {
+  static __device__ __forceinline__ int lane_id() {
+    int lane = threadIdx.x & 63;
+    if constexpr (FRESH) asm volatile("" : "+v"(lane));
+    return lane;
+  }
   typename Mfma<DT>::vec q[8];  // Q^T: dims 16 s + 8 half .. + 7 of the lane's query
   f32x16 acc[4];                // O^T: dim 32 t + 8 (i / 4) + 4 half + i % 4
   float base;                   // running maximum, log2 units
@@ -157,7 +166,7 @@ struct State {
   __device__ __forceinline__ void scores(const Rows& k, f32x16 (&c)[2]) {
     using M = Mfma<DT>;
     using vec = typename M::vec;
-    const int lane = threadIdx.x & 63, half = lane >> 5;
+    const int lane = lane_id(), half = lane >> 5;
     constexpr int kAhead = 4;   // K operands in flight
     vec kf[kAhead];
     auto read_k = [&](int n) {  // n = 2 s + kt
@@ -194,7 +203,7 @@ struct State {
   __device__ __forceinline__ void step(const f32x16 (&c)[2], const Rows& v, float k2) {
     using M = Mfma<DT>;
     using vec = typename M::vec;
-    const int lane = threadIdx.x & 63, half = lane >> 5;
+    const int lane = lane_id(), half = lane >> 5;
     float mx = c[0][0];
 #pragma unroll
     for (int i = 1; i < 32; ++i) mx = fmaxf(mx, c[i >> 4][i & 15]);
@@ -208,8 +217,8 @@ struct State {
     // 4 m .. + 3 (of the group's 16) of row 16 ks + 8 u + 4 half + j
     const int j = (lane & 15) >> 2, m = lane & 3, gi = (lane >> 4) & 1;
     const int low = 2 * gi + (m >> 1);
-    auto read_v = [&](int n) {   // n = 4 d + ks
-      const int d = n >> 2, ks = n & 3;
+    auto read_v = [&](int n) {   // n = 4 ks + d
+      const int d = n & 3, ks = n >> 2;
       s16x4v x[2];
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
@@ -220,38 +229,40 @@ struct State {
       }
       return __builtin_bit_cast(vec, __builtin_shufflevector(x[0], x[1], 0, 1, 2, 3, 4, 5, 6, 7));
     };
+    // P of the 16 keys of step ks, a quarter (two scores) at a time: the next
+    // step's between this one's MFMAs
+    uint32_t ph[2][4], pl[2][4];
+    auto quarter = [&](int ks, int e) {
+      const float p0 = __builtin_amdgcn_exp2f(fmaf(c[ks >> 1][8 * (ks & 1) + 2 * e], k2, -base));
+      const float p1 = __builtin_amdgcn_exp2f(fmaf(c[ks >> 1][8 * (ks & 1) + 2 * e + 1], k2, -base));
+      const uint32_t h = M::round2(p0, p1);
+      ph[ks & 1][e] = h;
+      den = M::sum2(h, den);
+      if constexpr (HILO) {
+        pl[ks & 1][e] = M::round2(p0 - M::widen(static_cast<uint16_t>(h)), p1 - M::widen(static_cast<uint16_t>(h >> 16)));
+        den = M::sum2(pl[ks & 1][e], den);
+      }
+    };
     constexpr int kAhead = 3;   // V operands in flight
     vec vf[kAhead];
-    uint32_t ph[16], pl[16];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const float p0 = __builtin_amdgcn_exp2f(fmaf(c[e >> 3][2 * (e & 7)], k2, -base));
-      const float p1 = __builtin_amdgcn_exp2f(fmaf(c[e >> 3][2 * (e & 7) + 1], k2, -base));
-      ph[e] = M::round2(p0, p1);
-      den = M::sum2(ph[e], den);
-      if constexpr (HILO) {
-        pl[e] = M::round2(p0 - M::widen(static_cast<uint16_t>(ph[e])), p1 - M::widen(static_cast<uint16_t>(ph[e] >> 16)));
-        den = M::sum2(pl[e], den);
-      }
-    }
-    acc[0] *= alpha;
 #pragma unroll
     for (int n = 0; n < kAhead; ++n) vf[n] = read_v(n);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) quarter(0, e);
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int n = 0; n < 16; ++n) {
       __builtin_amdgcn_sched_barrier(0);
-      const int d = n >> 2, ks = n & 3;
-      const vec vv = vf[n % kAhead];
-      acc[d] = M::run(vv, __builtin_bit_cast(vec, make_uint4(ph[4 * ks], ph[4 * ks + 1], ph[4 * ks + 2], ph[4 * ks + 3])),
-                      acc[d]);
-      if constexpr (HILO)
-        acc[d] = M::run(vv, __builtin_bit_cast(vec, make_uint4(pl[4 * ks], pl[4 * ks + 1], pl[4 * ks + 2], pl[4 * ks + 3])),
-                        acc[d]);
+      const int d = n & 3, ks = n >> 2;
+      const uint32_t* h = ph[ks & 1];
+      if (ks == 0) acc[d] *= alpha;
+      acc[d] = M::run(vf[n % kAhead], __builtin_bit_cast(vec, make_uint4(h[0], h[1], h[2], h[3])), acc[d]);
+      if constexpr (HILO) {
+        const uint32_t* l = pl[ks & 1];
+        acc[d] = M::run(vf[n % kAhead], __builtin_bit_cast(vec, make_uint4(l[0], l[1], l[2], l[3])), acc[d]);
+      }
       if (n + kAhead < 16) vf[n % kAhead] = read_v(n + kAhead);
-      if (d < 3)
-#pragma unroll
-        for (int i = 4 * ks; i < 4 * ks + 4; ++i) acc[d + 1][i] *= alpha;
+      if (ks < 3) quarter(ks + 1, d);
     }
     __builtin_amdgcn_s_setprio(0);
   }
@@ -261,7 +272,7 @@ struct State {
   template <class StoreFn>
   __device__ __forceinline__ void store(uint4* lds, StoreFn put) {
     using M = Mfma<DT>;
-    const int lane = threadIdx.x & 63, half = lane >> 5, qn = lane & 31;
+    const int lane = lane_id(), half = lane >> 5, qn = lane & 31;
     const float inv = 1.f / (den + __shfl_xor(den, 32, 64));
 #pragma unroll
     for (int d = 0; d < 4; ++d)
