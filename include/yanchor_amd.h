@@ -126,11 +126,14 @@ int yh_gdn_decode_fused(const void* proj, int64_t proj_stride, void* conv_state,
  *   final_state fp32 [n_seqs, HV, 128, V] (written)
  *   order NULL or int32 [n_seqs]: dispatch order of the sequences (longest
  *   first balances the grid); every sequence must appear once.
- *   workspace, workspace_bytes: unused (may be NULL / 0); every per-chunk
- *   quantity stays on chip.  yh_gdn_chunk_workspace_bytes returns 0.
+ *   workspace, workspace_bytes: 16-byte aligned scratch of at least
+ *   yh_gdn_chunk_workspace_bytes bytes, which is 0 unless few sequences would
+ *   leave most of the chip idle; without it (NULL / 0) every call takes the
+ *   one-launch form.  The results are the same bits either way.
  *   One launch: a workgroup per (sequence, value head) prepares each chunk
  *   (norms, decays, K K^T, Q K^T, the inverse of I + L) while it runs the
- *   state-dependent products of the previous one.
+ *   state-dependent products of the previous one.  With the workspace: one
+ *   launch prepares all chunks, a second one runs the state through them.
  */
 int yh_gdn_chunk_varlen(const void* q, const void* k, const void* v, const void* g, const void* beta,
                         const float* initial_state, float* final_state, void* o, const int32_t* cu_seqlens,

@@ -7,6 +7,8 @@ import torch
 
 from oracle import anchor as oracle_memory
 from oracle import glue
+from yanchor_amd import _native
+from yanchor_amd import gdn
 from yanchor_amd import independent_memory as im
 from yanchor_amd import layers
 
@@ -157,3 +159,33 @@ def test_memory_sequence_segments(gpu, cap, chunk, length, heads, groups, odd):
     for f in fields(st):
         assert torch.equal(getattr(packed_state, f.name), getattr(got_state, f.name)), f.name
     assert torch.equal(again, got[valid.to(gpu)])
+
+
+@pytest.mark.parametrize("lengths,h,hv,v,h0,gates", [
+    ([3001], 4, 4, 128, True, torch.float32),        # one tile a workgroup, a ragged last chunk
+    ([129, 0, 64, 700], 2, 8, 128, False, torch.bfloat16),   # an empty sequence, slots between chunks, GQA
+    ([500, 1], 3, 27, 128, True, torch.float32),     # two tiles a workgroup
+    ([191, 257], 16, 32, 64, True, torch.float32),   # 64 value columns
+])
+def test_gdn_few_sequences(gpu, lengths, h, hv, v, h0, gates):
+    """The same operations in the same order as the one-launch form: the same
+    bits as that form gives the same sequences among many."""
+    gen = torch.Generator().manual_seed(3)
+    n, copies = sum(lengths), -(-300 // (len(lengths) * hv * v // 32)) + 1
+    q, k = (torch.randn(1, n, h, 128, generator=gen).to(torch.bfloat16).to(gpu) for _ in range(2))
+    val = torch.randn(1, n, hv, v, generator=gen).to(torch.bfloat16).to(gpu)
+    g = torch.nn.functional.logsigmoid(torch.randn(1, n, hv, generator=gen) + 3).to(gates).to(gpu)
+    beta = torch.rand(1, n, hv, generator=gen).to(gates).to(gpu)
+    s0 = torch.randn(len(lengths), hv, 128, v, generator=gen).to(gpu) * 0.02 if h0 else None
+    need = _native.lib().yh_gdn_chunk_workspace_bytes
+    assert need(n, len(lengths), hv, v) > 0 and need(copies * n, copies * len(lengths), hv, v) == 0
+
+    def run(c):
+        x = [t.repeat(1, c, 1, 1) for t in (q, k, val)] + [t.repeat(1, c, 1) for t in (g, beta)]
+        return gdn.chunk_gated_delta_rule(*x[:3], g=x[3], beta=x[4], use_qk_l2norm_in_kernel=True,
+                                          initial_state=None if s0 is None else s0.repeat(c, 1, 1, 1),
+                                          output_final_state=True, cu_seqlens=_cu(lengths * c, gpu))
+    o, st = run(1)
+    many_o, many_st = run(copies)
+    assert torch.equal(o, many_o[:, :n]) and torch.equal(st, many_st[: len(lengths)])
+    assert torch.equal(o, many_o[:, -n:]) and torch.equal(st, many_st[-len(lengths):])

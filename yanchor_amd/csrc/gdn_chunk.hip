@@ -10,9 +10,9 @@
 //   S <- e^{G_last} S + K^T diag(e^{G_last - G}) v_new
 // with q, k L2-normalised (eps 1e-6 inside rsqrt) and q scaled.
 //
-// T and A = Q K^T o Gamma do not depend on the state S.  One kernel,
-// chunk_fused_kernel, runs one workgroup per (sequence, value head) that walks
-// the sequence's chunks.  Eight scan waves hold the 128 x V fp32 state in MFMA
+// T and A = Q K^T o Gamma do not depend on the state S.  chunk_fused_kernel
+// runs one workgroup per (sequence, value head) that walks the sequence's chunks
+// (few sequences: chunk_prep_kernel and chunk_scan_kernel below).  Eight scan waves hold the 128 x V fp32 state in MFMA
 // accumulators (wave w owns value columns 16w..16w+15) and run the
 // state-dependent products of chunk j - 1 (Q S and K S, v_new, o, the state
 // update, with S and v_new never leaving registers) while four prep waves
@@ -174,6 +174,12 @@ __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" :
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, const void* lds, int voff) {
   const unsigned m0v = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds)));
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" ::"s"(m0v), "v"(voff), "s"(r)
+               : "memory", "m0");
+}
+// The same for data that other workgroups read too.
+__device__ __forceinline__ void dma16_shared(__amdgpu_buffer_rsrc_t r, const void* lds, int voff) {
+  const unsigned m0v = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds)));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(m0v), "v"(voff), "s"(r)
                : "memory", "m0");
 }
 __device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t r, const void* lds, int voff) {
@@ -823,15 +829,297 @@ __global__ void __launch_bounds__((NW + kNP) * 64) chunk_fused_kernel(FusedArgs 
   }
 }
 
+// ---------------------------------------------------------------------------
+// Few sequences: a workgroup per (sequence, head) leaves most of the chip idle
+// and every chunk costs the whole chain of the six phases (5.6 us; 265 us for
+// one sequence of 3001 tokens, on 32 of 256 CUs).  What does not depend on the
+// state is then prepared for all chunks at once (chunk_prep_kernel), and the
+// scan, left with the state-dependent products, is spread over more waves
+// (chunk_scan_kernel): the state's columns do not meet, so a workgroup takes CT
+// of a head's 16-column tiles, and four waves share a tile, each with 16 of the
+// chunk's tokens and 32 of the state's rows; they meet in LDS three times a
+// chunk, for D = V - W' S, for v_new and for the state.  The same operations in
+// the same order as chunk_fused_kernel: the same bits.  (One wave a tile, with
+// nothing to exchange, takes 3.7 us a chunk: a serial chain of 104 MFMAs and
+// the splits into hi + lo.)
+//
+// Record of a (chunk slot, value head) in the workspace: T diag(beta) hi / lo,
+// A and the scalings, as they lie in LDS.  The slots of sequence n start at
+// cu[n] / 64 + n, which leaves each its ceil(length / 64).
+constexpr int kRecT = kC * 16, kRecA = kC * 8, kRecS = kC;   // 16-byte pieces
+constexpr int kRecord = kRecT + kRecA + kRecS;
+
+__device__ __forceinline__ int64_t first_slot(const int32_t* cu, int n) { return cu[n] / kC + n; }
+
+__global__ void __launch_bounds__(256) chunk_prep_kernel(FusedArgs a, uint4* ws) {
+  __shared__ FBuf Y;
+  __shared__ FPrep pp;
+  const int hv = blockIdx.x % a.HV, hk = hv / (a.HV / a.H);
+  const int64_t slot = blockIdx.x / a.HV;
+  int n = a.n_seqs - 1;
+  while (n > 0 && first_slot(a.cu, n) > slot) --n;
+  const int j = static_cast<int>(slot - first_slot(a.cu, n));
+  const int seqlen = a.cu[n + 1] - a.cu[n];
+  if (j * kC >= seqlen) return;   // a slot without a chunk
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, quad = lane >> 4;
+  const int64_t tok = a.cu[n] + static_cast<int64_t>(j) * kC;
+  const int Lp = min(kC, seqlen - j * kC);
+
+  fdma_q<0, 4>(Y, a, tok, Lp, hk);
+  fdma_k<0, 4>(Y, a, tok, Lp, hk);
+  fdma_g<0>(Y, a, tok, Lp, hv);
+  if (tid < 2 * 16 * 4) {  // A's halves in the upper blocks (0, 1) and (2, 3)
+    const int rr = tid >> 2, t = rr < 16 ? rr : 16 + rr, p = t < 16 ? (tid & 3) : 4 + (tid & 3);
+    reinterpret_cast<uint2*>(&Y.aqk[tpos(t, p)])[1] = make_uint2(0, 0);
+  }
+  dma_wait();
+  lds_barrier();
+
+  if (w == 3) {  // decay cumsum; lane t: token t
+    const int64_t gi = (tok + (lane < Lp ? lane : Lp - 1)) * a.HV + hv;
+    const float bt = lane < Lp ? gate_value(Y.gw[kC + lane], gi, a.beta_dt) : 0.f;
+    const float x = wave_prefix_sum(lane < Lp ? gate_value(Y.gw[lane], gi, a.g_dt) : 0.f);
+    pp.G[lane] = x;
+    pp.G2[lane] = x * 1.4426950408889634f;
+    pp.beta[lane] = bt;
+    if (lane == kWave - 1) pp.gl = x;
+  }
+  f32x4v kk[3], qk[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    if (w + 4 * i < 10) kq_tile(Y, pp, a, w + 4 * i, kk[i], qk[i], r16, quad);
+  lds_barrier();
+
+  if (w == 3) {
+    const float eg = expf(pp.G[lane]);
+    Y.scal[lane] = eg * pp.rqs[lane];
+    Y.scal[kC + lane] = pp.rk[lane] * expf(pp.gl - pp.G[lane]);
+    Y.scal[2 * kC + lane] = -eg * pp.rk[lane];
+    if (lane == 0) Y.scal[3 * kC] = expf(pp.gl);
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    if (w + 4 * i < 10) la_tile(Y, pp, w + 4 * i, kk[i], qk[i], r16, quad);
+  lds_barrier();
+
+  float* tf = Y.vt.t;
+  if (w == 0) inv_diag(Y.tt.l, tf);
+  lds_barrier();
+  f32x4v y0, y1;
+  if (w < 2) inv_level1(Y.tt.l, tf, w);
+  inv_level2_pre(Y.tt.l, tf, w, y0, y1);
+  lds_barrier();
+  inv_level2_fin(Y.tt.l, tf, w, y0, y1);
+  lds_barrier();
+#pragma unroll
+  for (int it = 0; it < 4; ++it) t_hilo(Y, tf, pp, (it * 256 + tid) * 4);
+  lds_barrier();
+
+  uint4* rec = ws + (slot * a.HV + hv) * kRecord;
+#pragma unroll
+  for (int it = 0; it < kRecT / 256; ++it) rec[it * 256 + tid] = Y.tt.p[it * 256 + tid];
+#pragma unroll
+  for (int it = 0; it < kRecA / 256; ++it) rec[kRecT + it * 256 + tid] = Y.aqk[it * 256 + tid];
+  if (tid < kRecS) rec[kRecT + kRecA + tid] = reinterpret_cast<const uint4*>(Y.scal)[tid];
+}
+
+template <int CT>
+struct __align__(16) ScanBuf {
+  uint4 q[kC * 16];     // as in FBuf
+  uint4 k[kC * 16];
+  uint4 p[kRecT];
+  uint4 aqk[kRecA];
+  float scal[4 * kC];
+  uint4 v[CT][kC * 2];  // V [t][16 columns], unswizzled
+};
+// Operands that the four waves of a tile hand each other, in the B layout:
+// state rows 32 ks .. + 31; D, v_new (scaled for the state update, and rounded
+// for the output) of tokens 32 ks .. + 31, where token tile mt is half mt % 2.
+struct __align__(16) ScanShare {
+  uint4 sh[4][kWave], sl[4][kWave];
+  uint4 dh[2][kWave], dl[2][kWave];
+  uint4 zh[2][kWave], zl[2][kWave];
+  uint4 vn[2][kWave];
+};
+static_assert(2 * sizeof(ScanBuf<2>) + 2 * sizeof(ScanShare) <= 160 * 1024, "scan LDS");
+
+template <int V, int CT>
+__global__ void __launch_bounds__(CT * 256) chunk_scan_kernel(FusedArgs a, const uint4* ws) {
+  __shared__ ScanBuf<CT> bufs[2];
+  __shared__ ScanShare shares[CT];
+  constexpr int kParts = V / (16 * CT), NWV = 4 * CT;
+  const int hv = blockIdx.x % a.HV, hk = hv / (a.HV / a.H);   // the parts of a head: one XCD where 8 divides HV
+  const int rest = blockIdx.x / a.HV, part = rest % kParts, sidx = rest / kParts;
+  const int n = a.order ? a.order[sidx] : sidx;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, quad = lane >> 4, rq4 = quad * 4;
+  const int tl = w >> 2, mw = w & 3;             // the wave's tile; its token tile and its 32 state rows
+  const int ct = part * CT + tl;
+  const int64_t seq0 = a.cu[n], slot0 = first_slot(a.cu, n);
+  const int seqlen = a.cu[n + 1] - a.cu[n];
+  const int nch = (seqlen + kC - 1) / kC;
+  ScanShare& sx = shares[tl];
+
+  auto load = [&](ScanBuf<CT>& X, int j) {
+    const int64_t tok = seq0 + static_cast<int64_t>(j) * kC;
+    const int Lc = min(kC, seqlen - j * kC);
+    const int ks = a.H * kK * 2, vs = a.HV * V * 2;
+    const auto rq = chunk_rsrc(a.q + (tok * a.H + hk) * kK, Lc, ks, kK * 2);
+    const auto rk = chunk_rsrc(a.k + (tok * a.H + hk) * kK, Lc, ks, kK * 2);
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(ws) + ((slot0 + j) * a.HV + hv) * kRecord, 0,
+                                                      kRecord * 16, 0x00020000);
+#pragma unroll
+    for (int bl = w; bl < 16; bl += NWV) {
+      const int row = 4 * bl + (lane >> 4), off = row * ks + (((lane & 15) ^ swz_qk(row)) & 15) * 16;
+      dma16_shared(rk, &X.k[64 * bl], off);
+      dma16_shared(rq, &X.q[64 * bl], off);
+      dma16_shared(rw, &X.p[64 * bl], (64 * bl + lane) * 16);
+    }
+#pragma unroll
+    for (int bl = w; bl < 9; bl += NWV)
+      dma16_shared(rw, bl < 8 ? static_cast<const void*>(&X.aqk[64 * bl]) : X.scal, (kRecT + 64 * bl + lane) * 16);
+    if (mw >= 2) {   // the tile's 32 token rows of V
+      const auto rv = chunk_rsrc(a.v + (tok * a.HV + hv) * V, Lc, vs, V * 2);
+      dma16_shared(rv, &X.v[tl][64 * (mw - 2)], (32 * (mw - 2) + (lane >> 1)) * vs + (2 * ct + (lane & 1)) * 16);
+    }
+  };
+
+  // S[q][i]: state row state_row(2 mw + q, quad, i), value column vcol
+  f32x4v S[2];
+  const int vcol = 16 * ct + r16;
+  const int64_t sbase = (static_cast<int64_t>(n) * a.HV + hv) * kK;
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[q][i] = a.h0 ? a.h0[(sbase + state_row(2 * mw + q, quad, i)) * V + vcol] : 0.f;
+  auto share_state = [&]() {
+    bf16x8_t hi, lo;
+    pack_b(S[0], S[1], hi, lo);
+    sx.sh[mw][lane] = __builtin_bit_cast(uint4, hi);
+    sx.sl[mw][lane] = __builtin_bit_cast(uint4, lo);
+  };
+  share_state();
+  if (nch > 0) load(bufs[0], 0);
+  dma_wait();
+  wait_vmem();   // (known to the compiler: it places no wait for the state at the loop head)
+  lds_barrier();
+#pragma unroll 1
+  for (int j = 0; j < nch; ++j) {
+    const ScanBuf<CT>& X = bufs[j & 1];
+    if (j + 1 < nch) load(bufs[(j + 1) & 1], j + 1);
+    // (Q S)^T and K S of the wave's tokens
+    f32x4v qs = {0.f, 0.f, 0.f, 0.f}, ps = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const bf16x8_t bh = __builtin_bit_cast(bf16x8_t, sx.sh[ks][lane]);
+      const bf16x8_t bl = __builtin_bit_cast(bf16x8_t, sx.sl[ks][lane]);
+      const bf16x8_t ak = lds_k(X.k, 16 * mw + r16, ks, quad);
+      ps = mfma(ak, bh, ps);
+      ps = mfma(ak, bl, ps);
+      qs = mfma(bh, lds_k(X.q, 16 * mw + r16, ks, quad), qs);
+    }
+    // D = V - diag(e^G rk) K S, as hi + lo
+    uint32_t hi[2], lo[2];
+    {
+      const uint2* vp = reinterpret_cast<const uint2*>(&X.v[tl][(16 * mw + rq4 + (r16 >> 2)) * 2]) + (r16 & 3);
+      const uint2 vw = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4v*)vp));
+      const float4 sc = *reinterpret_cast<const float4*>(&X.scal[2 * kC + 16 * mw + rq4]);
+      split2(fmaf(ps[0], sc.x, __uint_as_float(vw.x << 16)), fmaf(ps[1], sc.y, __uint_as_float(vw.x & 0xffff0000u)),
+             hi[0], lo[0]);
+      split2(fmaf(ps[2], sc.z, __uint_as_float(vw.y << 16)), fmaf(ps[3], sc.w, __uint_as_float(vw.y & 0xffff0000u)),
+             hi[1], lo[1]);
+    }
+    reinterpret_cast<uint2*>(&sx.dh[mw >> 1][lane])[mw & 1] = make_uint2(hi[0], hi[1]);
+    reinterpret_cast<uint2*>(&sx.dl[mw >> 1][lane])[mw & 1] = make_uint2(lo[0], lo[1]);
+    lds_barrier();
+    // v_new of the wave's tokens = T diag(beta) D
+    f32x4v u = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      if (ks == 0 || mw >= 2) {
+        const bf16x8_t dh = __builtin_bit_cast(bf16x8_t, sx.dh[ks][lane]);
+        const bf16x8_t dl = __builtin_bit_cast(bf16x8_t, sx.dl[ks][lane]);
+        const bf16x8_t th = __builtin_bit_cast(bf16x8_t, X.p[thi(16 * mw + r16, 4 * ks + quad)]);
+        const bf16x8_t tlo_ = __builtin_bit_cast(bf16x8_t, X.p[tlo(16 * mw + r16, 4 * ks + quad)]);
+        u = mfma(th, dh, u);
+        u = mfma(th, dl, u);
+        y = mfma(tlo_, dh, y);
+      }
+    }
+    const f32x4v vn = u + y;
+    {
+      const float4 sc = *reinterpret_cast<const float4*>(&X.scal[kC + 16 * mw + rq4]);
+      split2(vn[0] * sc.x, vn[1] * sc.y, hi[0], lo[0]);
+      split2(vn[2] * sc.z, vn[3] * sc.w, hi[1], lo[1]);
+    }
+    typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+    reinterpret_cast<uint2*>(&sx.zh[mw >> 1][lane])[mw & 1] = make_uint2(hi[0], hi[1]);
+    reinterpret_cast<uint2*>(&sx.zl[mw >> 1][lane])[mw & 1] = make_uint2(lo[0], lo[1]);
+    reinterpret_cast<uint2*>(&sx.vn[mw >> 1][lane])[mw & 1] =
+        __builtin_bit_cast(uint2, __builtin_convertvector(vn, bf16x4_t));
+    lds_barrier();
+    // S <- e^{G_last} S + K^T z, the wave's 32 rows
+    const float egl = X.scal[3 * kC];
+    bf16x8_t zh[2], zl[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      zh[ks] = __builtin_bit_cast(bf16x8_t, sx.zh[ks][lane]);
+      zl[ks] = __builtin_bit_cast(bf16x8_t, sx.zl[ks][lane]);
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      f32x4v sv = S[q] * egl;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        const bf16x8_t ak = lds8t_key(X.k, 32 * ks, 2 * mw + q, lane);
+        sv = mfma(ak, zh[ks], sv);
+        sv = mfma(ak, zl[ks], sv);
+      }
+      S[q] = sv;
+    }
+    share_state();
+    // o^T of the wave's tokens.  The buffer store drops rows past the sequence by
+    // itself, so exactly one vector memory operation lies behind the copies of
+    // chunk j + 1 and the wait below leaves it in flight.
+    const int t = 16 * mw + r16, os = a.HV * V * 2, Ls = min(kC, seqlen - j * kC);
+    const auto ro = __builtin_amdgcn_make_buffer_rsrc(
+        a.o + ((seq0 + static_cast<int64_t>(j) * kC) * a.HV + hv) * V, 0, (Ls - 1) * os + V * 2, 0x00020000);
+    f32x4v acc = qs * X.scal[t];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      if (ks == 0 || mw >= 2) acc = mfma(__builtin_bit_cast(bf16x8_t, sx.vn[ks][lane]), lds_t(X.aqk, t, ks, quad), acc);
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, __builtin_convertvector(acc, bf16x4_t)), ro,
+                                          t * os + (16 * ct + 4 * quad) * 2, 0, 0);
+    asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
+    lds_barrier();   // chunk j + 1 has arrived; X is consumed; the state is shared
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a.ht[(sbase + state_row(2 * mw + q, quad, i)) * V + vcol] = S[q][i];
+}
+
+// The split form pays while its scan, 4 workgroups a head of 128 columns, runs
+// in one round (one workgroup a CU) and a sequence has a few chunks on average.
+// Two sequences x 32 heads: 123 us against 167; four of 4000 tokens: 417 against
+// 361.  One sequence of 300 tokens: 50 against 60; of 50: 43 against 40.
+bool split_form(int64_t total_tokens, int64_t n_seqs, int64_t HV, int64_t V) {
+  return n_seqs * HV * (V / 32) <= 256 && total_tokens > 128 * n_seqs;
+}
+
+template <int V, int CT>
+void launch_scan(const FusedArgs& f, const uint4* ws, hipStream_t st) {
+  hipLaunchKernelGGL((chunk_scan_kernel<V, CT>), dim3(static_cast<unsigned>(f.n_seqs * f.HV * (V / (16 * CT)))),
+                     dim3(CT * 256), 0, st, f, ws);
+}
+
 }  // namespace
 }  // namespace yh
 
 extern "C" int64_t yh_gdn_chunk_workspace_bytes(int64_t total_tokens, int64_t n_seqs, int64_t HV, int64_t V) {
-  (void)total_tokens;
-  (void)n_seqs;
-  (void)HV;
-  (void)V;
-  return 0;  // the one-pass kernel keeps every per-chunk quantity on chip
+  if (n_seqs <= 0 || HV <= 0 || V <= 0 || !yh::split_form(total_tokens, n_seqs, HV, V)) return 0;
+  return (total_tokens / yh::kC + n_seqs) * HV * yh::kRecord * 16;
 }
 
 extern "C" int yh_gdn_chunk_varlen(const void* q, const void* k, const void* v, const void* g, const void* beta,
@@ -841,8 +1129,6 @@ extern "C" int yh_gdn_chunk_varlen(const void* q, const void* k, const void* v, 
                                    int use_qk_l2norm, int qkv_dtype, int g_dtype, int beta_dtype, void* workspace,
                                    int64_t workspace_bytes, yh_stream_t stream) {
   using namespace yh;
-  (void)workspace;
-  (void)workspace_bytes;
   YH_CHECK_ARG(n_seqs >= 0 && total_tokens >= 0 && H > 0 && HV > 0 && HV % H == 0, "gdn_chunk: bad sizes");
   YH_CHECK_ARG(K == 128, "gdn_chunk: K must be 128 (got %lld)", (long long)K);
   YH_CHECK_ARG(V == 64 || V == 128, "gdn_chunk: V must be 64 or 128 (got %lld)", (long long)V);
@@ -862,6 +1148,23 @@ extern "C" int yh_gdn_chunk_varlen(const void* q, const void* k, const void* v, 
   FusedArgs f{static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), g,
               beta, cu_seqlens, order, initial_state, final_state, static_cast<uint16_t*>(o), (int)n_seqs, (int)H,
               (int)HV, scale, use_qk_l2norm ? 1 : 0, g_dtype, beta_dtype};
+  const int64_t need = yh_gdn_chunk_workspace_bytes(total_tokens, n_seqs, HV, V);
+  const int64_t slots = total_tokens / kC + n_seqs;
+  if (need > 0 && workspace && workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+      slots * HV < (1LL << 24)) {
+    uint4* ws = static_cast<uint4*>(workspace);
+    hipLaunchKernelGGL(chunk_prep_kernel, dim3(static_cast<unsigned>(slots * HV)), dim3(256), 0, st, f, ws);
+    YH_CHECK_LAUNCH("gdn_chunk prep");
+    // one tile a workgroup where that still is one round (151 against 161 us for
+    // one sequence of 3001 tokens x 32 heads)
+    const bool one = n_seqs * HV * (V / 16) <= 256;
+    if (V == 128 && one) launch_scan<128, 1>(f, ws, st);
+    else if (V == 128) launch_scan<128, 2>(f, ws, st);
+    else if (one) launch_scan<64, 1>(f, ws, st);
+    else launch_scan<64, 2>(f, ws, st);
+    YH_CHECK_LAUNCH("gdn_chunk scan");
+    return YH_OK;
+  }
   const dim3 grid(static_cast<unsigned>(n_seqs * HV));
   if (V == 128)
     hipLaunchKernelGGL(chunk_fused_kernel<8>, grid, dim3((8 + kNP) * 64), 0, st, f);

@@ -119,8 +119,9 @@ def chunk_gated_delta_rule(query, key, value, g=None, beta=None, scale=None, ini
     own call, T > 1) as B packed sequences of T tokens.  Other shapes, or
     ``force_recurrent=True``, run the token-recurrent kernel over each
     sequence.  ``lengths`` (host ints, one per sequence) lets the chunk
-    kernel start the longest sequences first.  The chunk kernel needs no
-    scratch memory, so concurrent calls on different streams are independent.
+    kernel start the longest sequences first.  Scratch memory, which only
+    calls of few sequences need, belongs to the call, so concurrent calls on
+    different streams are independent.
     """
     if g is None or beta is None:
         raise ValueError("chunk_gated_delta_rule needs g and beta")
@@ -162,12 +163,15 @@ def chunk_gated_delta_rule(query, key, value, g=None, beta=None, scale=None, ini
         h0 = None if initial_state is None else initial_state.contiguous()
         state = torch.empty(n, hv, kd, vd, device=dev, dtype=torch.float32)
         order = None
-        if lengths is not None:  # longest sequences first balances the grid
+        if lengths is not None and n > 1:  # longest sequences first balances the grid
             order = torch.tensor(sorted(range(n), key=lambda i: -int(lengths[i])), dtype=torch.int32,
                                  device=dev)
+        # scratch for the few-sequences form; none otherwise
+        need = N.lib().yh_gdn_chunk_workspace_bytes(total, n, hv, vd)
+        ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
         N.call("yh_gdn_chunk_varlen", q.data_ptr(), k.data_ptr(), v.data_ptr(), g_.data_ptr(), be.data_ptr(),
                N.ptr(h0), state.data_ptr(), o.data_ptr(), cu.data_ptr(), N.ptr(order), n, total, h, hv, kd, vd, sc,
-               int(bool(use_qk_l2norm_in_kernel)), N.code(q), N.code(g_), N.code(be), None, 0, N.stream_of(q))
+               int(bool(use_qk_l2norm_in_kernel)), N.code(q), N.code(g_), N.code(be), N.ptr(ws), need, N.stream_of(q))
         return o, (state if output_final_state else None)
     if initial_state is None:
         state = torch.zeros(n, hv, kd, vd, device=dev, dtype=torch.float32)
