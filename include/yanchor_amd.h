@@ -752,8 +752,10 @@ int yh_linear_reduce(const float* part, void* out, int64_t out_stride, int64_t M
  *   conv_w  [channels, 4]
  *   out     [total_tokens, channels] = bf16(silu(sum_j x(t-3+j) w[c, j])),
  *           fp32 taps in the order of the decode prologue (yh_gdn_decode_prep)
- * dtype: bf16.
+ * dtype: bf16, alone or | YH_CONV_PLANES(p): out is then p column groups apart,
+ * [p, total_tokens, channels / p].
  */
+#define YH_CONV_PLANES(p) ((p) << 8)
 int yh_conv_prefill(const void* proj, int64_t proj_stride, void* window, const void* conv_w,
                     const int32_t* cu_seqlens, int64_t n_seqs, int64_t total_tokens, int64_t channels, void* out,
                     int dtype, yh_stream_t stream);

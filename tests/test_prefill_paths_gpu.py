@@ -34,7 +34,10 @@ def test_conv_prefill_runs(gpu, lengths, channels, pad):
     window = torch.randn(len(lengths), 3, channels, generator=g).to(torch.bfloat16)
     w = (torch.randn(channels, 4, generator=g) * 0.5).to(torch.bfloat16)
     win = window.to(gpu)
-    out = layers.conv_prefill(proj.to(gpu), win, w.to(gpu), _cu(lengths, gpu), channels).cpu()
+    args = (proj.to(gpu), win, w.to(gpu), _cu(lengths, gpu), channels)
+    planes = layers.conv_prefill(args[0], window.to(gpu), *args[2:], planes=4).cpu()
+    out = layers.conv_prefill(*args).cpu()
+    assert torch.equal(planes, out.view(n, 4, channels // 4).transpose(0, 1))
     off = 0
     for r, length in enumerate(lengths):
         y, new = glue.causal_conv1d_prefill(proj[off: off + length, :channels], window[r], w)

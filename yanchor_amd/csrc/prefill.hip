@@ -55,8 +55,8 @@ struct ConvArgs {
   const uint16_t* window;
   const uint16_t* w;
   const int32_t* cu;
-  uint16_t* y;
-  int64_t C;
+  uint16_t* y;         // [C / Cp, total, Cp]
+  int64_t C, Cp;
   int nseq;
 };
 
@@ -108,7 +108,8 @@ __global__ void __launch_bounds__(256) conv_prefill_kernel(ConvArgs a, int64_t t
   int64_t s = a.cu[r], e = a.cu[r + 1];
   if (n0 >= e) return;   // tokens outside every piece
   const T* src = reinterpret_cast<const T*>(a.proj + c);
-  const int64_t sp = a.P / VEC, sc = a.C / VEC;
+  const int64_t sp = a.P / VEC, sc = a.C / VEC, yc = a.Cp / VEC, plane = c / a.Cp;
+  T* dst = reinterpret_cast<T*>(a.y + plane * total * a.Cp + (c - plane * a.Cp));
 
   float wt[4][VEC];
 #pragma unroll
@@ -172,7 +173,7 @@ __global__ void __launch_bounds__(256) conv_prefill_kernel(ConvArgs a, int64_t t
         h[1][v] = h[2][v];
         h[2][v] = cur;
       }
-      reinterpret_cast<T*>(a.y + c)[n * sc] = Ch::pack(y);
+      dst[n * yc] = Ch::pack(y);
     }
   }
 }
@@ -409,15 +410,19 @@ extern "C" int yh_conv_prefill(const void* proj, int64_t proj_stride, void* wind
   using namespace yh;
   YH_CHECK_ARG(n_seqs >= 0 && total_tokens >= 0 && channels > 0 && proj_stride >= channels,
                "conv_prefill: bad sizes");
+  const int64_t planes = dtype >> 8 > 0 ? dtype >> 8 : 1;
+  dtype &= 0xff;
   YH_CHECK_ARG(dtype == YH_BF16, "conv_prefill: activations must be bfloat16");
+  YH_CHECK_ARG(channels % planes == 0, "conv_prefill: planes must divide the channels");
   if (n_seqs == 0) return YH_OK;
   YH_CHECK_ARG(proj && window && conv_w && cu_seqlens && (out || total_tokens == 0), "conv_prefill: null pointer");
   YH_CHECK_ARG(total_tokens < (1ll << 31) && n_seqs < (1ll << 31), "conv_prefill: sizes too large");
   hipStream_t st = static_cast<hipStream_t>(stream);
   ConvArgs c{static_cast<const uint16_t*>(proj), proj_stride, static_cast<const uint16_t*>(window),
-             static_cast<const uint16_t*>(conv_w), cu_seqlens, static_cast<uint16_t*>(out), channels, (int)n_seqs};
+             static_cast<const uint16_t*>(conv_w), cu_seqlens, static_cast<uint16_t*>(out), channels,
+             channels / planes, (int)n_seqs};
   // 16-byte channel groups where every row of every tensor keeps them aligned
-  const bool vec = channels % 8 == 0 && proj_stride % 8 == 0 && aligned16(proj) && aligned16(window) &&
+  const bool vec = channels / planes % 8 == 0 && proj_stride % 8 == 0 && aligned16(proj) && aligned16(window) &&
                    aligned16(out) && (reinterpret_cast<uintptr_t>(conv_w) & 7) == 0;
   const int64_t per_block = 256 * (vec ? 8 : 1);
   const unsigned cb = static_cast<unsigned>((channels + per_block - 1) / per_block);

@@ -460,42 +460,48 @@ def linear(x, w, split_k=None, residual=None, defer=False):
 # Refill prefill of packed, ragged prompt pieces (cu_seqlens), each continuing
 # its sequence's caches.
 
-def _cu(cu_seqlens, device, total):
+def _cu(cu_seqlens, device, total, starts=None, ring_rows=None, ring_batch=0):
     """cu_seqlens (host or device) as int32 on the device, checked on the
-    host (a prefill is not captured, so the copy is cheap): non-decreasing,
-    from >= 0 to <= total, so no kernel reads past the packed tokens.  The
-    small per-piece vectors (offsets, starts, ring rows) may come from the
-    host; the activations and caches must be device tensors."""
+    host: non-decreasing, from >= 0 to <= total, so no kernel reads past the
+    packed tokens.  With ``starts`` and ``ring_rows``, one entry per piece,
+    these too: starts >= 0, rows inside the ring.  A prefill is not captured,
+    so a copy to the host is possible, but it waits for the stream: everything
+    that is checked comes in one.  The small per-piece vectors may come from
+    the host; the activations and caches must be device tensors.  Returns (cu,
+    its values on the host, starts, ring_rows)."""
     cu = cu_seqlens.to(device=device, dtype=torch.int32).contiguous()
     if cu.ndim != 1 or cu.numel() < 1:
         raise ValueError("cu_seqlens must be a 1-D offset vector")
-    h = cu.cpu()
-    if int(h[0]) != 0 or int(h[-1]) > total or bool((h[1:] < h[:-1]).any()):
+    m, st, rr = cu.numel(), None, None
+    if starts is None:
+        h = cu.tolist()
+    else:
+        st = starts.to(device=device, dtype=torch.int64).contiguous()
+        rr = ring_rows.to(device=device, dtype=torch.int64).contiguous()
+        h = torch.cat((cu, st.reshape(-1), rr.reshape(-1))).tolist()
+    if h[0] != 0 or h[m - 1] > total or any(h[i + 1] < h[i] for i in range(m - 1)):
         raise ValueError("cu_seqlens must be non-decreasing offsets from 0 within the packed tokens")
-    return cu
+    if starts is not None:
+        if st.shape != (m - 1,) or rr.shape != (m - 1,):
+            raise ValueError("starts / ring_rows must hold one entry per piece")
+        if m > 1 and (min(h[m: 2 * m - 1]) < 0 or max(h[2 * m - 1:]) >= ring_batch):
+            raise ValueError("starts must be >= 0 and ring rows inside the ring")
+    return cu, h[:m], st, rr
 
 
-def _pieces(starts, ring_rows, r, ring_batch, device):
-    st = starts.to(device=device, dtype=torch.int64).contiguous()
-    rr = ring_rows.to(device=device, dtype=torch.int64).contiguous()
-    if st.shape != (r,) or rr.shape != (r,):
-        raise ValueError("starts / ring_rows must hold one entry per piece")
-    if r and (int(st.min()) < 0 or int(rr.max()) >= ring_batch):
-        raise ValueError("starts must be >= 0 and ring rows inside the ring")
-    return st, rr
-
-
-def conv_prefill(proj, window, conv_w, cu_seqlens, channels):
+def conv_prefill(proj, window, conv_w, cu_seqlens, channels, planes=1):
     """The GDN layer's causal conv1d + SiLU over packed prompt pieces
     (the causal-conv1d prefill of the CUDA backend, modeling_yanchor.py:
     392-407): proj [N, >= channels] bf16 (the conv inputs are its first
     ``channels`` columns, any row stride), window [R, 3, channels] bf16, the
     inputs before each piece (zeros for a fresh sequence), updated IN PLACE
-    to the last three inputs; conv_w [channels, 4].  Returns [N, channels]."""
+    to the last three inputs; conv_w [channels, 4].  Returns [N, channels], or
+    with ``planes`` > 1 its column groups apart, [planes, N, channels / planes]
+    (q, k and v as the recurrence reads them, without a copy of each)."""
     _bf16(proj, window, conv_w)
     n = proj.shape[0]
     dev = N.require_device(proj, window, conv_w)
-    cu = _cu(cu_seqlens, dev, n)
+    cu, offsets, _, _ = _cu(cu_seqlens, dev, n)
     r = cu.numel() - 1
     if proj.ndim != 2 or proj.stride(1) != 1 or proj.shape[1] < channels:
         raise ValueError("proj must be [N, >= channels] with unit column stride")
@@ -503,19 +509,24 @@ def conv_prefill(proj, window, conv_w, cu_seqlens, channels):
         raise ValueError("window must be contiguous [R, 3, channels]")
     if conv_w.shape != (channels, 4) or not conv_w.is_contiguous():
         raise ValueError("conv_w must be contiguous [channels, 4]")
-    if int(cu[-1]) != n:
+    if offsets[-1] != n:
         raise ValueError("cu_seqlens must cover every packed token")
-    out = torch.empty(n, channels, dtype=proj.dtype, device=dev)
+    if planes < 1 or channels % planes:
+        raise ValueError("planes must divide the channels")
+    out = torch.empty((n, channels) if planes == 1 else (planes, n, channels // planes), dtype=proj.dtype, device=dev)
     N.call("yh_conv_prefill", proj.data_ptr(), proj.stride(0), window.data_ptr(), conv_w.data_ptr(), cu.data_ptr(),
-           r, n, channels, out.data_ptr(), N.BF16, N.stream_of(proj))
+           r, n, channels, out.data_ptr(), N.BF16 | (planes << 8 if planes > 1 else 0), N.stream_of(proj))
     return out
 
 
 def prefill_tiles(lengths, tokens_per_tile, device):
     """(piece, first token) int32 [n_tiles, 2] of the tiles of
     ``tokens_per_tile`` tokens that cover pieces of the given host lengths."""
-    tiles = [(r, t) for r, n in enumerate(lengths) for t in range(0, int(n), tokens_per_tile)]
-    return torch.tensor(tiles, dtype=torch.int32).reshape(-1, 2).to(device)
+    n = torch.as_tensor([int(x) for x in lengths], dtype=torch.int64)
+    count = (n + tokens_per_tile - 1).clamp_min(0) // tokens_per_tile
+    piece = torch.repeat_interleave(torch.arange(n.numel()), count)
+    first = (torch.arange(piece.numel()) - (count.cumsum(0) - count)[piece]) * tokens_per_tile
+    return torch.stack((piece, first), 1).to(torch.int32).to(device)
 
 
 def _rows(x, name):
@@ -547,12 +558,11 @@ def swa_prefill(q, k, v, cu_seqlens, starts, ring_k, ring_v, ring_rows, *, gate=
     if not ring_k.is_contiguous() or not ring_v.is_contiguous() or ring_k.dtype != q.dtype:
         raise ValueError("ring tensors must be contiguous in the query dtype")
     dev = N.require_device(q, k, v, ring_k, ring_v, gate)
-    cu = _cu(cu_seqlens, dev, n)
+    cu, offsets, st, rr = _cu(cu_seqlens, dev, n, starts, ring_rows, ring_k.shape[0])
     r = cu.numel() - 1
-    st, rr = _pieces(starts, ring_rows, r, ring_k.shape[0], dev)
     if 64 % (h // g):
         raise ValueError("query heads per KV head must divide 64")
-    lengths = (cu[1:] - cu[:-1]).tolist()
+    lengths = [b - a for a, b in zip(offsets, offsets[1:])]
     if tiles is None:
         tiles = prefill_tiles(lengths, 64 // (h // g), dev)
     else:
@@ -591,9 +601,8 @@ def ring_fill(k, v, cu_seqlens, starts, ring_rows, ring_k, ring_v, ring_pos):
         if not t.is_contiguous():
             raise ValueError("ring tensors must be contiguous")
     dev = N.require_device(k, v, ring_k, ring_v, ring_pos)
-    cu = _cu(cu_seqlens, dev, n)
+    cu, _, st, rr = _cu(cu_seqlens, dev, n, starts, ring_rows, ring_k.shape[0])
     r = cu.numel() - 1
-    st, rr = _pieces(starts, ring_rows, r, ring_k.shape[0], dev)
     k, v = _rows(k, "k"), _rows(v, "v")
     N.call("yh_ring_fill", k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), rr.data_ptr(), st.data_ptr(),
            cu.data_ptr(), r, n, ring_k.data_ptr(), ring_v.data_ptr(), ring_pos.data_ptr(), g, d, ring_k.shape[2],

@@ -251,6 +251,9 @@ class HipOps:
                                                output_final_state=True, use_qk_l2norm_in_kernel=True,
                                                cu_seqlens=cu_seqlens, lengths=lengths)
 
+    def conv_prefill_planes(self, proj, window, conv_w, cu_seqlens, channels, planes):
+        return self.layers.conv_prefill(proj, window, conv_w, cu_seqlens, channels, planes=planes)
+
     def conv_prefill(self, proj, window, conv_w, cu_seqlens, channels, lengths):
         if proj.dtype != torch.bfloat16:
             return TorchGlue.conv_prefill(proj, window, conv_w, cu_seqlens, channels, lengths)
@@ -860,7 +863,7 @@ class Model:
                 src = torch.tensor([off[i] + lens[i] - 1 for i in ends], device=dev)
                 last.index_copy_(0, torch.tensor(ends, device=dev), h.index_select(0, src))
         xn = self.ops.rmsnorm(last, self.final_norm, c.rms_eps)
-        logits = F.linear(xn, self.lm_head).float()
+        logits = self.ops.linear(xn, self.lm_head, self.lm_head_packed).float()
         return logits, tmp.cache_tensors()
 
     def _prefill_piece(self, tmp, tokens, starts, lens):
@@ -877,15 +880,18 @@ class Model:
         starts_t = torch.tensor(starts, dtype=torch.int64, device=dev)
         cos, sin = rope_tables(pos, c)
         h = self.embed[tokens]
+        xn = ops.rmsnorm(h, self.layers[0]["in_norm"], c.rms_eps)
         for i, L in enumerate(self.layers):
-            xn = ops.rmsnorm(h, L["in_norm"], c.rms_eps)
             if L["kind"] == "gdn":
                 delta = self._gdn_prefill(i, L, tmp, xn, cu, lens)
             else:
                 delta = self._attn_prefill(i, L, tmp, xn, h, cos, sin, cu, starts_t, lens)
-            h = h + delta
-            h = h + self._mlp(L, ops.rmsnorm(h, L["post_norm"], c.rms_eps))
-        return h
+            # each residual add in the norm that follows it, as in the decode step
+            xn, h = ops.rmsnorm(delta, L["post_norm"], c.rms_eps, residual=h)
+            mlp = self._mlp(L, xn)
+            if i + 1 < len(self.layers):
+                xn, h = ops.rmsnorm(mlp, self.layers[i + 1]["in_norm"], c.rms_eps, residual=h)
+        return h + mlp
 
     def _gdn_prefill(self, i, L, tmp, xn, cu, lens):
         """GDN mixer over packed pieces: conv (continuing the window), the
@@ -895,11 +901,14 @@ class Model:
         n = xn.shape[0]
         hk, dk, hv, dv = c.gdn_heads_k, c.gdn_dk, c.gdn_heads_v, c.gdn_dv
         proj = F.linear(xn, L["w_in"])                                      # [N, qkv | z | b | a]
-        mixed = ops.conv_prefill(proj, tmp.conv_state[i], L["conv_w"], cu, c.conv_dim, lens)
+        if hk * dk == hv * dv and proj.dtype == torch.bfloat16 and hasattr(ops, "conv_prefill_planes"):
+            # q, k, v as the recurrence reads them
+            q, k, v = ops.conv_prefill_planes(proj, tmp.conv_state[i], L["conv_w"], cu, c.conv_dim, 3)
+        else:
+            q, k, v = ops.conv_prefill(proj, tmp.conv_state[i], L["conv_w"], cu, c.conv_dim, lens).split(
+                (hk * dk, hk * dk, hv * dv), 1)
         _, _, beta, g = self._gdn_split(L, proj)
-        q = mixed[:, : hk * dk].reshape(1, n, hk, dk)
-        k = mixed[:, hk * dk: 2 * hk * dk].reshape(1, n, hk, dk)
-        v = mixed[:, 2 * hk * dk:].reshape(1, n, hv, dv)
+        q, k, v = q.reshape(1, n, hk, dk), k.reshape(1, n, hk, dk), v.reshape(1, n, hv, dv)
         # the chunked recurrence runs from and to float32; a float16 store rounds once a piece
         o, st = ops.gdn_prefill(q, k, v, g[None], beta[None], cu, lens, initial_state=tmp.gdn_state[i].float())
         tmp.gdn_state[i].copy_(st)
