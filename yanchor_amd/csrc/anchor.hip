@@ -246,11 +246,11 @@ template <int DT, int R, bool SKIP> constexpr int read_occupancy() {
   return DT == YH_F32 ? 2 : SKIP ? (R == 1 ? 4 : 3) : R == 4 ? 3 : 2;
 }
 
-template <int DT, int D, int R, bool SINK, int BS, bool SKIP>
-__global__ void __launch_bounds__((read_waves<R>() * 64))
+template <int DT, int D, int R, bool SINK, int BS, bool SKIP, int W = read_waves<R>()>
+__global__ void __launch_bounds__((W * 64))
 __attribute__((amdgpu_waves_per_eu(read_occupancy<DT, R, SKIP>(), read_occupancy<DT, R, SKIP>())))
 anchor_read_kernel(ReadArgs a) {
-  constexpr int kReadWaves = read_waves<R>();
+  constexpr int kReadWaves = W;
   constexpr int kReadThreads = kReadWaves * 64;
   constexpr int LPR = D / 8;
   constexpr int RPI = kWave / LPR;
@@ -707,7 +707,28 @@ int launch_read_r(int R, const ReadArgs& a, hipStream_t st) {
     case 3: hipLaunchKernelGGL((anchor_read_kernel<DT, D, 1, SINK, kSkipBS, SINK>), grid, b1, 0, st, a); break;
     case 4: hipLaunchKernelGGL((anchor_read_kernel<DT, D, 2, SINK, BS, false>), grid, b2, 0, st, a); break;
     case 5: hipLaunchKernelGGL((anchor_read_kernel<DT, D, 2, SINK, kSkipBS, SINK>), grid, b2, 0, st, a); break;
-    case 8: hipLaunchKernelGGL((anchor_read_kernel<DT, D, 4, SINK, kR4BS, false>), grid, b4, 0, st, a); break;
+    case 8: {
+      // Few memories leave CUs idle while two waves walk a memory's blocks one
+      // after the other: up to one memory a CU takes as many waves as a CU
+      // holds (window ring) or as its 16 blocks feed (256 slots), up to three a
+      // CU four waves.  1024-slot ring and 256-slot memory, 8 memories a row,
+      // us with two waves -> with these: 1 row 68 and 20 -> 24 and 10, 32 rows
+      // 69 and 21 -> 30 and 12, 64 rows 78 and 24 -> 51 and 17, 96 rows 91 and 26
+      // -> 76 and 24; 128 rows' memory 29 -> 33.  A memory of a few blocks has
+      // nothing to share out.
+      constexpr int kMany = DT == YH_F32 ? 8 : 12;
+      const int64_t memories = static_cast<int64_t>(a.B) * a.G;
+      const int w = a.KC < 64 || memories > 768 ? 2 : memories > 256 ? 4 : a.KC > 256 ? kMany : 6;
+      if (w == kMany)
+        hipLaunchKernelGGL((anchor_read_kernel<DT, D, 4, SINK, kR4BS, false, kMany>), grid, dim3(kMany * 64), 0, st, a);
+      else if (w == 6)
+        hipLaunchKernelGGL((anchor_read_kernel<DT, D, 4, SINK, kR4BS, false, 6>), grid, dim3(6 * 64), 0, st, a);
+      else if (w == 4)
+        hipLaunchKernelGGL((anchor_read_kernel<DT, D, 4, SINK, kR4BS, false, 4>), grid, dim3(4 * 64), 0, st, a);
+      else
+        hipLaunchKernelGGL((anchor_read_kernel<DT, D, 4, SINK, kR4BS, false>), grid, b4, 0, st, a);
+      break;
+    }
     default: set_error("anchor_read: heads per group must be 1, 2 or 4 (got %d)", R); return YH_ERR_INVALID;
   }
   YH_CHECK_LAUNCH("anchor_read");
