@@ -696,18 +696,30 @@ namespace {
 //
 // One workgroup per row.  Every draw is a selection "the first element, in a
 // given order, whose inclusive cumulative weight reaches t": the elements are
-// ordered by a 64-bit key K (descending), (value key << 32 | ~index) for value
-// order (larger value first, lower index first on equal values) or ~index
-// for vocabulary order.  K* is found 4 bits at a time from the top: a pass
-// over the row sums the weight of the elements that share the bits fixed so
-// far into 16 buckets of the next digit, and the largest digit whose
-// cumulative weight (with everything above) reaches t is kept.  Weights are
-// counts (for the top-k cut) or probabilities as 2^62 fixed-point integers,
-// so every sum is exact and independent of summation order.  The row is
-// re-read on every pass (from L2 / the Infinity Cache after the first).
+// ordered by a key E (descending), 32 value bits (larger value first) over 20
+// bits of ~index (lower index first on equal values) for value order, or the 20
+// index bits alone for vocabulary order.  E* is found 12 bits at a time from the
+// top: a pass over the row adds the weight of the elements that share the bits
+// fixed so far to 4096 buckets of the next digit in LDS, and the largest digit
+// whose cumulative weight (with everything above) reaches t is kept; once at
+// most kFullList elements are left, one more pass lists them and they are ranked
+// against each other.  Weights are counts (for the top-k cut) or probabilities
+// as 2^62 fixed-point integers, so every sum is exact and independent of
+// summation order.  The two draws of the value order (the top_p cut and the
+// token) share the first digit's buckets.
+//
+// Bound by the exponentials and the fixed-point conversions of a row on one CU
+// (a third of the time each for S and the first digit).  4-bit digits in
+// registers (13 passes a draw, 16 conditional 64-bit additions an element) took
+// 2259 us at 30 rows x 151936 bf16, top_p 0.95; this takes 418 us (top_p 1, in
+// vocabulary order: 574 and 254; 160 rows: 3293 and 558).
 constexpr int kFullThreads = 1024;
 constexpr int kFullWaves = kFullThreads / kWave;
-constexpr int kFan = 16;
+constexpr int kFullDigit = 12;
+constexpr int kFullBuckets = 1 << kFullDigit;
+constexpr int kFullPer = kFullBuckets / kFullThreads;
+constexpr int kFullList = 512;
+constexpr int kFullBatch = 8;               // elements a thread has in flight
 constexpr double kMassOne = 4611686018427387904.0;  // 2^62: fixed-point probability 1
 
 struct FullArgs {
@@ -722,43 +734,30 @@ struct FullArgs {
   float penalty, temperature, top_p;
 };
 
+struct FullHist {
+  unsigned long long weight[kFullBuckets];
+  uint32_t count[kFullBuckets];
+};
 struct FullShared {
-  uint64_t part[kFullWaves][kFan];
-  uint32_t cpart[kFullWaves][kFan];
-  uint64_t bucket[kFan];
-  uint32_t bcount[kFan];
+  FullHist first, next;   // the first digit's buckets of the masses; any other's
+  unsigned long long lkey[kFullList], lweight[kFullList];
+  uint64_t wsum[kFullWaves];
   double dpart[kFullWaves];
   float fpart[kFullWaves];
+  int last[kFullWaves], top[kFullWaves];
+  int nlist;
+  int digit;              // the selection's results
+  uint32_t dcount;
+  uint64_t above, dweight, key, incl;
 };
 
-__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += shfl_xor_u64(v, off);
-  return v;
-}
-__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-  return v;
-}
 __device__ __forceinline__ double wave_sum_f64(double v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
   return v;
 }
 
-// Score of element i with the presence penalty applied (before temperature).
-template <int DT>
-__device__ __forceinline__ float full_value(const FullArgs& a, const char* row, const uint8_t* srow, int i) {
-  uint32_t bits;
-  if constexpr (DT == YH_F32) bits = *reinterpret_cast<const uint32_t*>(row + static_cast<int64_t>(i) * 4);
-  else bits = *reinterpret_cast<const uint16_t*>(row + static_cast<int64_t>(i) * 2);
-  float x = decode_elem<DT>(bits);
-  if (srow && srow[i]) x = x - a.penalty;
-  return x;
-}
-
-// Selection state of one row: the candidate set is K >= lo; weights are
+// Selection state of one row: the candidate set is E >= lo; weights are
 // masses (mass) or counts; masses need the row's tempered maximum mt and
 // the candidate set's sum S of exp(x / T - mt).
 struct FullRow {
@@ -769,121 +768,213 @@ struct FullRow {
   double scale;  // 2^62 / S: fixed-point mass per unit of exp(x / T - mt)
 };
 
-__device__ __forceinline__ uint64_t full_key(const FullArgs& a, float x, int i) {
-  return a.vocab_order ? static_cast<uint64_t>(0xffffffffu - static_cast<uint32_t>(i)) : ckey(x, static_cast<uint32_t>(i));
+// f(score of element i with the presence penalty applied (before temperature),
+// i, whether there is an element i) for i = tid, tid + 1024, .. in order,
+// kFullBatch loads ahead; every lane of a wave makes every call.
+template <int DT, class F>
+__device__ __forceinline__ void full_each(const FullArgs& a, const FullRow& r, F f) {
+  for (int base = 0; base < a.V; base += kFullThreads * kFullBatch) {
+    const int i0 = base + threadIdx.x;
+    uint32_t bits[kFullBatch];
+    bool seen[kFullBatch];
+#pragma unroll
+    for (int e = 0; e < kFullBatch; ++e) {
+      const int64_t i = min(i0 + e * kFullThreads, a.V - 1);
+      if constexpr (DT == YH_F32) bits[e] = *reinterpret_cast<const uint32_t*>(r.row + i * 4);
+      else bits[e] = *reinterpret_cast<const uint16_t*>(r.row + i * 2);
+      seen[e] = r.srow != nullptr && r.srow[i];
+    }
+#pragma unroll
+    for (int e = 0; e < kFullBatch; ++e) {
+      const int i = i0 + e * kFullThreads;
+      float x = decode_elem<DT>(bits[e]);
+      if (seen[e]) x = x - a.penalty;
+      f(x, i, i < a.V);
+    }
+  }
 }
 
-template <int DT>
+__device__ __forceinline__ uint64_t full_key(const FullArgs& a, float x, int i) {
+  const uint64_t at = 0xfffffu - static_cast<uint32_t>(i);   // index < 2^20
+  return a.vocab_order ? at : (static_cast<uint64_t>(okey(x)) << 20) | at;
+}
+
 __device__ __forceinline__ uint64_t full_mass(const FullArgs& a, const FullRow& r, float x) {
   const float xt = x / a.temperature;
   return static_cast<uint64_t>(static_cast<double>(expf(xt - r.mt)) * r.scale);
 }
 
-// The largest K* among candidates with W(K >= K*) >= t (t >= 1), and
-// W(K >= K*) in *incl.  Bits from `top` up are fixed to `prefix` (the bits of
-// ~index above bit 19, all ones for an index below 2^20).  If t exceeds the
-// candidates' total weight the smallest candidate key is returned.
+// The buckets of the digit of `width` bits at `pos` of the candidates whose
+// bits above it are `prefix`.
 template <int DT, bool MASS>
-__device__ uint64_t full_select(const FullArgs& a, const FullRow& r, uint64_t t, int top, uint64_t prefix,
-                                uint64_t* incl, FullShared& sh) {
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
-  uint64_t above = 0;  // weight of candidates with a key above every key of the current prefix
-  for (int pos = top - 4; pos >= 0; pos -= 4) {
-    if (!a.vocab_order && pos == 28) {  // ~index bits 31..20: all ones (index < 2^20)
-      prefix = (prefix << 12) | 0xfffull;
-      pos = 16;
-    }
-    uint64_t acc[kFan];
-    uint32_t cnt[kFan];
+__device__ void full_buckets(const FullArgs& a, const FullRow& r, FullHist& h, uint64_t prefix, int pos, int width) {
+  for (int c = threadIdx.x; c < kFullBuckets; c += kFullThreads) {
+    h.weight[c] = 0;
+    h.count[c] = 0;
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & (kWave - 1);
+  const bool share = a.vocab_order || pos + width < 52;
+  full_each<DT>(a, r, [&](float x, int i, bool in) {
+    const uint64_t E = full_key(a, x, i);
+    in = in && E >= r.lo && (E >> (pos + width)) == prefix;
+    const uint64_t who = __ballot(in);
+    if (who == 0) return;
+    const int d = static_cast<int>((E >> pos) & ((1u << width) - 1));
+    uint64_t w = 0;
+    if (MASS && in) w = full_mass(a, r, x);
+    // a wave whose elements all share the digit (neighbours in vocabulary order,
+    // tied scores past the first digit) adds once: 64 additions to one bucket
+    // would queue
+    const int d0 = share ? __shfl(d, __builtin_ctzll(who), kWave) : 0;
+    if (share && __ballot(in && d == d0) == who) {
+      if constexpr (MASS) {
 #pragma unroll
-    for (int c = 0; c < kFan; ++c) {
-      acc[c] = 0;
-      cnt[c] = 0;
-    }
-    for (int i = tid; i < a.V; i += kFullThreads) {
-      const float x = full_value<DT>(a, r.row, r.srow, i);
-      const uint64_t K = full_key(a, x, i);
-      if (K < r.lo || (pos + 4 < 64 && (K >> (pos + 4)) != prefix)) continue;
-      const int d = static_cast<int>((K >> pos) & 0xf);
-      const uint64_t w = MASS ? full_mass<DT>(a, r, x) : 1ull;
-#pragma unroll
-      for (int c = 0; c < kFan; ++c) {
-        acc[c] += d == c ? w : 0ull;
-        cnt[c] += d == c ? 1u : 0u;
+        for (int off = 32; off > 0; off >>= 1) w += shfl_xor_u64(w, off);
       }
-    }
-#pragma unroll
-    for (int c = 0; c < kFan; ++c) {
-      const uint64_t s = wave_sum_u64(acc[c]);
-      const uint32_t n = wave_sum_u32(cnt[c]);
       if (lane == 0) {
-        sh.part[wv][c] = s;
-        sh.cpart[wv][c] = n;
+        if constexpr (MASS) atomicAdd(&h.weight[d0], static_cast<unsigned long long>(w));
+        atomicAdd(&h.count[d0], static_cast<uint32_t>(__popcll(who)));
       }
+    } else if (in) {
+      if constexpr (MASS) atomicAdd(&h.weight[d], static_cast<unsigned long long>(w));
+      atomicAdd(&h.count[d], 1u);
     }
-    __syncthreads();
-    if (tid < kFan) {
-      uint64_t s = 0;
-      uint32_t n = 0;
-      for (int w = 0; w < kFullWaves; ++w) {
-        s += sh.part[w][tid];
-        n += sh.cpart[w][tid];
-      }
-      sh.bucket[tid] = s;
-      sh.bcount[tid] = n;
-    }
-    __syncthreads();
-    // largest digit whose cumulative weight reaches t; past the total, the
-    // smallest non-empty digit
-    int dsel = -1, last = 0;
-    uint64_t cum = above, cum_last = above;
-    for (int c = kFan - 1; c >= 0; --c) {
-      if (sh.bcount[c]) {
-        last = c;
-        cum_last = cum;
-      }
-      if (cum + sh.bucket[c] >= t && sh.bcount[c]) {
-        dsel = c;
-        break;
-      }
-      cum += sh.bucket[c];
-    }
-    if (dsel < 0) {
-      dsel = last;
-      cum = cum_last;
-    }
-    const uint64_t w_sel = sh.bucket[dsel];
-    const uint32_t n_sel = sh.bcount[dsel];
-    __syncthreads();
-    above = cum;
-    prefix = (prefix << 4) | static_cast<uint64_t>(dsel);
-    if (n_sel == 1 && pos > 0) {
-      // a single element left: its key is the largest key under the prefix
-      uint64_t best = 0;
-      for (int i = tid; i < a.V; i += kFullThreads) {
-        const float x = full_value<DT>(a, r.row, r.srow, i);
-        const uint64_t K = full_key(a, x, i);
-        if (K >= r.lo && (K >> pos) == prefix) best = K > best ? K : best;
-      }
+  });
+  __syncthreads();
+}
+
+// Inclusive prefix sum over the workgroup in thread order, and the total.
+__device__ __forceinline__ uint64_t full_scan(uint64_t v, uint64_t* total, FullShared& sh) {
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
 #pragma unroll
-      for (int off = 32; off > 0; off >>= 1) {
-        const uint64_t y = shfl_xor_u64(best, off);
-        best = y > best ? y : best;
-      }
-      if (lane == 0) sh.part[wv][0] = best;
-      __syncthreads();
-      uint64_t k = 0;
-      for (int w = 0; w < kFullWaves; ++w) k = sh.part[w][0] > k ? sh.part[w][0] : k;
-      __syncthreads();
-      *incl = above + w_sel;
-      return k;
+  for (int off = 1; off < kWave; off <<= 1) {
+    const uint64_t y = __shfl_up(static_cast<unsigned long long>(v), off, kWave);
+    if (lane >= off) v += y;
+  }
+  __syncthreads();  // wsum free
+  if (lane == kWave - 1) sh.wsum[wv] = v;
+  __syncthreads();
+  uint64_t all = 0;
+  for (int w = 0; w < kFullWaves; ++w) {
+    if (w < wv) v += sh.wsum[w];
+    all += sh.wsum[w];
+  }
+  *total = all;
+  return v;
+}
+
+// The largest digit of the buckets whose cumulative weight, `above` included,
+// reaches t; past the total, the smallest that is not empty; for t = 0 (no mass
+// anywhere: a row whose S is NaN) the largest that is not empty.  Into
+// sh.digit, dcount, dweight and above (the weight above the digit).
+template <bool MASS>
+__device__ void full_digit(const FullHist& h, uint64_t above, uint64_t t, FullShared& sh) {
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+  uint64_t w[kFullPer], sum = 0;
+  int last = -1;            // this thread's smallest digit that is not empty, as a place from the top
+  int top = kFullBuckets;   // and its largest
+#pragma unroll
+  for (int e = 0; e < kFullPer; ++e) {
+    const int c = kFullBuckets - 1 - (tid * kFullPer + e);
+    w[e] = MASS ? h.weight[c] : h.count[c];
+    if (h.count[c]) {
+      last = tid * kFullPer + e;
+      top = min(top, last);
     }
-    if (pos == 0) {
-      *incl = above + w_sel;
-      return prefix;
+    sum += w[e];
+  }
+  uint64_t total;
+  const uint64_t incl = full_scan(sum, &total, sh);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    last = max(last, __shfl_xor(last, off, kWave));
+    top = min(top, __shfl_xor(top, off, kWave));
+  }
+  if (lane == 0) {
+    sh.last[wv] = last;
+    sh.top[wv] = top;
+  }
+  if (above + incl >= t && above + incl - sum < t) {
+    uint64_t cum = above + incl - sum;
+#pragma unroll
+    for (int e = 0; e < kFullPer; ++e) {
+      if (cum < t && cum + w[e] >= t) {
+        sh.digit = kFullBuckets - 1 - (tid * kFullPer + e);
+        sh.above = cum;
+      }
+      cum += w[e];
     }
   }
-  *incl = above;
+  __syncthreads();
+  if (tid == 0) {
+    if (t == 0 || above + total < t) {
+      int place = 0, first = kFullBuckets - 1;
+      for (int v = 0; v < kFullWaves; ++v) {
+        place = max(place, sh.last[v]);
+        first = min(first, sh.top[v]);
+      }
+      sh.digit = kFullBuckets - 1 - (t == 0 ? first : place);
+      sh.above = t == 0 ? above : above + total - (MASS ? h.weight[sh.digit] : h.count[sh.digit]);
+    }
+    sh.dweight = MASS ? h.weight[sh.digit] : h.count[sh.digit];
+    sh.dcount = h.count[sh.digit];
+  }
+  __syncthreads();
+}
+
+// The largest E* among candidates with W(E >= E*) >= t (t >= 1), and
+// W(E >= E*) in *incl.  If t exceeds the candidates' total weight the smallest
+// candidate key is returned.  first: sh.first holds the first digit's buckets.
+template <int DT, bool MASS>
+__device__ uint64_t full_select(const FullArgs& a, const FullRow& r, uint64_t t, bool first, uint64_t* incl,
+                                FullShared& sh) {
+  const int tid = threadIdx.x;
+  uint64_t above = 0, prefix = 0;
+  for (int pos = a.vocab_order ? 20 : 52; pos > 0;) {
+    const int width = min(pos, kFullDigit);
+    pos -= width;
+    if (!first) full_buckets<DT, MASS>(a, r, sh.next, prefix, pos, width);
+    full_digit<MASS>(first ? sh.first : sh.next, above, t, sh);
+    first = false;
+    above = sh.above;
+    prefix = (prefix << width) | static_cast<uint64_t>(sh.digit);
+    const uint32_t left = sh.dcount;
+    if (pos == 0) {
+      *incl = above + sh.dweight;
+      return prefix;
+    }
+    if (left > kFullList) continue;
+    // the elements left, then each one's cumulative weight
+    if (tid == 0) sh.nlist = 0;
+    __syncthreads();
+    full_each<DT>(a, r, [&](float x, int i, bool in) {
+      const uint64_t E = full_key(a, x, i);
+      if (!in || E < r.lo || (E >> pos) != prefix) return;
+      const int at = atomicAdd(&sh.nlist, 1);
+      sh.lkey[at] = E;
+      sh.lweight[at] = MASS ? full_mass(a, r, x) : 1ull;
+    });
+    __syncthreads();
+    if (tid < static_cast<int>(left)) {
+      const uint64_t mine = sh.lkey[tid], w = sh.lweight[tid];
+      uint64_t cum = above;
+      bool smallest = true, largest = true;
+      for (uint32_t j = 0; j < left; ++j) {
+        const uint64_t o = sh.lkey[j];
+        if (o >= mine) cum += sh.lweight[j];
+        else smallest = false;
+        largest &= o <= mine;
+      }
+      if (t == 0 ? largest : (cum >= t && cum - w < t) || (smallest && cum < t)) {
+        sh.key = mine;
+        sh.incl = cum;
+      }
+    }
+    __syncthreads();
+    *incl = sh.incl;
+    return sh.key;
+  }
   return prefix;
 }
 
@@ -899,7 +990,9 @@ __global__ void __launch_bounds__(kFullThreads) sample_full_kernel(FullArgs a) {
   // row maximum of the scores (the top of the value order; its tempered
   // value is the softmax shift torch uses, division being monotone)
   float m = -INFINITY;
-  for (int i = tid; i < a.V; i += kFullThreads) m = fmaxf(m, full_value<DT>(a, r.row, r.srow, i));
+  full_each<DT>(a, r, [&](float x, int, bool in) {
+    if (in) m = fmaxf(m, x);
+  });
   m = wave_max(m);
   if (lane == 0) sh.fpart[wv] = m;
   __syncthreads();
@@ -911,15 +1004,14 @@ __global__ void __launch_bounds__(kFullThreads) sample_full_kernel(FullArgs a) {
   uint64_t incl = 0;
   // top-k cut (1 < k < V, value order): the k-th largest key bounds the candidates
   if (!a.vocab_order && a.top_k > 1 && a.top_k < a.V)
-    r.lo = full_select<DT, false>(a, r, static_cast<uint64_t>(a.top_k), 64, 0ull, &incl, sh);
+    r.lo = full_select<DT, false>(a, r, static_cast<uint64_t>(a.top_k), false, &incl, sh);
 
   // S = sum of exp(x / T - mt) over the candidates (fixed order: per thread,
   // then the wave butterfly, then the waves in order)
   double s = 0.0;
-  for (int i = tid; i < a.V; i += kFullThreads) {
-    const float x = full_value<DT>(a, r.row, r.srow, i);
-    if (full_key(a, x, i) >= r.lo) s += static_cast<double>(expf(x / a.temperature - r.mt));
-  }
+  full_each<DT>(a, r, [&](float x, int i, bool in) {
+    if (in && full_key(a, x, i) >= r.lo) s += static_cast<double>(expf(x / a.temperature - r.mt));
+  });
   s = wave_sum_f64(s);
   if (lane == 0) sh.dpart[wv] = s;
   __syncthreads();
@@ -928,18 +1020,12 @@ __global__ void __launch_bounds__(kFullThreads) sample_full_kernel(FullArgs a) {
   __syncthreads();
   r.scale = kMassOne / s;
 
-  // total fixed-point mass of the candidates
+  // the first digit's buckets, and with them the total fixed-point mass
+  full_buckets<DT, true>(a, r, sh.first, 0ull, a.vocab_order ? 20 - kFullDigit : 52 - kFullDigit, kFullDigit);
   uint64_t tot = 0;
-  for (int i = tid; i < a.V; i += kFullThreads) {
-    const float x = full_value<DT>(a, r.row, r.srow, i);
-    if (full_key(a, x, i) >= r.lo) tot += full_mass<DT>(a, r, x);
-  }
-  tot = wave_sum_u64(tot);
-  if (lane == 0) sh.part[wv][0] = tot;
-  __syncthreads();
-  tot = 0;
-  for (int w = 0; w < kFullWaves; ++w) tot += sh.part[w][0];
-  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < kFullPer; ++e) tot += sh.first.weight[tid * kFullPer + e];
+  full_scan(tot, &tot, sh);
 
   const uint32_t id = static_cast<uint32_t>(a.ids[b]);
   const uint32_t st = static_cast<uint32_t>(a.steps ? a.steps[b] : a.step);
@@ -951,23 +1037,17 @@ __global__ void __launch_bounds__(kFullThreads) sample_full_kernel(FullArgs a) {
     uint64_t t = c < 1.0 ? 1ull : static_cast<uint64_t>(c);
     return t > hi ? hi : t;
   };
-  uint64_t key;
-  if (a.vocab_order) {
-    // first index whose cumulative probability reaches u * total; the index
-    // bits above bit 19 are ~index's all-ones
-    key = full_select<DT, true>(a, r, at_least(static_cast<double>(u) * static_cast<double>(tot), tot), 20,
-                                0xfffull, &incl, sh);
-  } else {
-    // last kept element: the first whose inclusive mass reaches top_p (so
-    // every element before it has an exclusive mass below top_p); then the
-    // draw inside the kept mass
-    full_select<DT, true>(a, r, at_least(static_cast<double>(a.top_p) * static_cast<double>(tot), tot), 64, 0ull,
-                          &incl, sh);
-    const uint64_t kept = incl;
-    key = full_select<DT, true>(a, r, at_least(static_cast<double>(u) * static_cast<double>(kept), kept), 64, 0ull,
-                                &incl, sh);
+  // the mass to reach: of everything in vocabulary order; in value order of
+  // what is kept, up to the first element whose inclusive mass reaches top_p
+  // (so every element before it has an exclusive mass below top_p)
+  uint64_t kept = tot;
+  if (!a.vocab_order) {
+    full_select<DT, true>(a, r, at_least(static_cast<double>(a.top_p) * static_cast<double>(tot), tot), true, &incl, sh);
+    kept = incl;
   }
-  if (tid == 0) a.out[b] = static_cast<int64_t>(0xffffffffu - static_cast<uint32_t>(key & 0xffffffffu));
+  const uint64_t key = full_select<DT, true>(
+      a, r, at_least(static_cast<double>(u) * static_cast<double>(kept), kept), true, &incl, sh);
+  if (tid == 0) a.out[b] = static_cast<int64_t>(0xfffffu - static_cast<uint32_t>(key & 0xfffffu));
 }
 
 // Both phases of the sampler with the candidate lists in `workspace`; the
