@@ -74,8 +74,7 @@ struct Chan<8> {
   static __device__ __forceinline__ T pack(const float (&y)[8]) {
     uint32_t w[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      w[i] = static_cast<uint32_t>(f32_to_bf16(y[2 * i])) | (static_cast<uint32_t>(f32_to_bf16(y[2 * i + 1])) << 16);
+    for (int i = 0; i < 4; ++i) w[i] = attn::Mfma<YH_BF16>::round2(y[2 * i], y[2 * i + 1]);
     return make_uint4(w[0], w[1], w[2], w[3]);
   }
 };
@@ -95,7 +94,8 @@ constexpr int kConvBatch = 4;  // rows in flight per thread
 // rows a run) in 16-byte accesses, four rows ahead of their use.  One token
 // and one channel a thread (2-byte accesses, every row loaded four times, a
 // sequence search a workgroup) took 976 us at 64 pieces of 17,400 tokens x
-// 12288 channels (871 MB); this takes 290 us with the host's checks.
+// 12288 channels (871 MB); this takes 247 us with the
+// host's checks.
 template <int VEC>
 __global__ void __launch_bounds__(256) conv_prefill_kernel(ConvArgs a, int64_t total, int run) {
   using Ch = Chan<VEC>;
@@ -125,7 +125,9 @@ __global__ void __launch_bounds__(256) conv_prefill_kernel(ConvArgs a, int64_t t
       for (int j = 0; j < 4; ++j) wt[j][i] = bf16_to_f32(a.w[(c + i) * 4 + j]);
     }
   }
-  float h[3][VEC];   // the inputs before the current token
+  // the inputs of kConvBatch tokens behind the three before them: token i of a
+  // batch reads h[i .. i + 3], so nothing moves but the last three a batch
+  float h[kConvBatch + 3][VEC];
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
     const int64_t u = n0 - s - 3 + j;
@@ -151,30 +153,32 @@ __global__ void __launch_bounds__(256) conv_prefill_kernel(ConvArgs a, int64_t t
         s = a.cu[r];
         e = a.cu[r + 1];
       }
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) h[i + 3][v] = Ch::f32(x[i], v);
       if (n < s) continue;
       if (n == s) {
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
           const T x0 = reinterpret_cast<const T*>(a.window + c)[(static_cast<int64_t>(r) * 3 + j) * sc];
 #pragma unroll
-          for (int v = 0; v < VEC; ++v) h[j][v] = Ch::f32(x0, v);
+          for (int v = 0; v < VEC; ++v) h[i + j][v] = Ch::f32(x0, v);
         }
       }
       float y[VEC];
 #pragma unroll
       for (int v = 0; v < VEC; ++v) {
-        const float cur = Ch::f32(x[i], v);
-        float acc = h[0][v] * wt[0][v];
-        acc = fmaf(h[1][v], wt[1][v], acc);
-        acc = fmaf(h[2][v], wt[2][v], acc);
-        acc = fmaf(cur, wt[3][v], acc);
+        float acc = h[i][v] * wt[0][v];
+        acc = fmaf(h[i + 1][v], wt[1][v], acc);
+        acc = fmaf(h[i + 2][v], wt[2][v], acc);
+        acc = fmaf(h[i + 3][v], wt[3][v], acc);
         y[v] = silu(acc);
-        h[0][v] = h[1][v];
-        h[1][v] = h[2][v];
-        h[2][v] = cur;
       }
       dst[n * yc] = Ch::pack(y);
     }
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) h[j][v] = h[kConvBatch + j][v];
   }
 }
 
