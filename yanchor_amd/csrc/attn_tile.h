@@ -22,7 +22,7 @@
 // product between the MFMAs of the step before; a raised wave priority around
 // the MFMAs, so that they run under the other wave's vector work; no mask code on
 // tiles where every key is live.  Six waves a workgroup (three a SIMD, 168
-// registers) spill and take 1.7 times as long.  The denominator sums the
+// registers) take 1.4 times as long even with the addresses re-formed a tile.  The denominator sums the
 // rounded P that the value product sees (two at a time, v_dot2), so the
 // rounding of a dominant probability cancels in the quotient.  (A running
 // maximum that lags the scores by up to 2^8 and leaves out most rescalings was
