@@ -12,8 +12,8 @@
 //
 // Query head h belongs to group h / (H / G).  Per (b, block, g) the C * H/G
 // query rows share one gathered set of CAP key/value rows, so the read is a
-// small dense attention: S^T = K Q^T and O^T = V^T P^T on 16x16x32 MFMA, with
-// an online softmax whose running max starts at 0 and denominator at 1 (the
+// small dense attention: S^T = K Q^T and O^T = V^T P^T on MFMA, with an
+// online softmax whose running max starts at 0 and denominator at 1 (the
 // sink logit 0 with value 0).  As in the reference, P enters the PV product as
 // a hi + lo pair of 16-bit values, so the product keeps fp32 accuracy.
 //

@@ -29,8 +29,8 @@
 // force (the `read_refs` of modeling_yanchor.py:248), and rewrites the scores,
 // positions and pending scores of the state in place; anchor_seq_commit_kernel
 // then copies the key / value rows of the final memory and of the new pending
-// tokens out of the assembled sources (modeling_yanchor.py:256-274) and
-// advances count / total.
+// tokens from where they are (modeling_yanchor.py:256-274) and advances count /
+// total.
 #include "anchor_source.h"
 
 namespace yh {
@@ -127,7 +127,8 @@ __device__ __forceinline__ int sort_candidates(uint64_t (*key)[kSortMax], uint16
 }
 
 // Bound by LDS latency (about ten dependent reads a merge level) at one
-// workgroup a CU.
+// workgroup a CU.  32 rows x 8 groups of 2048 tokens: 38 us, where merging one
+// block after the other into the memory took 195.
 __global__ void __launch_bounds__(kSortThreads) anchor_prefix_kernel(PrefixArgs a) {
   __shared__ uint64_t key[2][kSortMax];
   __shared__ uint16_t idx[2][kSortMax];

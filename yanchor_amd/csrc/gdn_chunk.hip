@@ -1105,7 +1105,8 @@ __global__ void __launch_bounds__(CT * 256) chunk_scan_kernel(FusedArgs a, const
 // Two sequences x 32 heads: 123 us against 167; four of 4000 tokens: 417 against
 // 361.  One sequence of 300 tokens: 50 against 60; of 50: 43 against 40.
 bool split_form(int64_t total_tokens, int64_t n_seqs, int64_t HV, int64_t V) {
-  return n_seqs * HV * (V / 32) <= 256 && total_tokens > 128 * n_seqs;
+  return n_seqs * HV * (V / 32) <= 256 && total_tokens > 128 * n_seqs &&
+         (total_tokens / kC + n_seqs) * HV * kRecord * 16 <= (1LL << 31);   // scratch of at most 2 GiB
 }
 
 template <int V, int CT>
