@@ -316,12 +316,12 @@ __device__ __forceinline__ void dma_rows(uint4* dst, __amdgpu_buffer_rsrc_t r, i
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t chunk_rsrc(const uint16_t* base, int Lc, int stride, int row_bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, (Lc - 1) * stride + row_bytes, 0x00020000);
 }
-template <int W0, int NWV>
-__device__ __forceinline__ void fdma_q(FBuf& b, const FusedArgs& a, int64_t tok0, int Lc, int hk) {
+template <int W0, int NWV, class B>
+__device__ __forceinline__ void fdma_q(B& b, const FusedArgs& a, int64_t tok0, int Lc, int hk) {
   dma_rows<true, W0, NWV>(b.q, chunk_rsrc(a.q + (tok0 * a.H + hk) * kK, Lc, a.H * kK * 2, kK * 2), a.H * kK * 2, 16);
 }
-template <int W0, int NWV>
-__device__ __forceinline__ void fdma_k(FBuf& b, const FusedArgs& a, int64_t tok0, int Lc, int hk) {
+template <int W0, int NWV, class B>
+__device__ __forceinline__ void fdma_k(B& b, const FusedArgs& a, int64_t tok0, int Lc, int hk) {
   dma_rows<true, W0, NWV>(b.k, chunk_rsrc(a.k + (tok0 * a.H + hk) * kK, Lc, a.H * kK * 2, kK * 2), a.H * kK * 2, 16);
 }
 template <int V, int W0, int NWV>
@@ -331,8 +331,8 @@ __device__ __forceinline__ void fdma_v(FBuf& b, const FusedArgs& a, int64_t tok0
 }
 // The gate words of chunk (tok0, Lc), by waves W0 (g) and W0 + 1 (beta); rows
 // past Lc repeat the last row's words (masked on use).
-template <int W0>
-__device__ __forceinline__ void fdma_g(FBuf& b, const FusedArgs& a, int64_t tok0, int Lc, int hv) {
+template <int W0, class B>
+__device__ __forceinline__ void fdma_g(B& b, const FusedArgs& a, int64_t tok0, int Lc, int hv) {
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) - W0;
   if (w == 0 || w == 1) {
     const void* src = w == 0 ? a.g : a.beta;
@@ -414,7 +414,8 @@ __device__ __forceinline__ void inv_level2_fin(const float* l, float* t, int u, 
 
 // Elements e .. e + 3 (row e / 64) of T diag(beta) as bf16 hi / lo; blocks
 // the products read as zeros are written as zeros.
-__device__ __forceinline__ void t_hilo(FBuf& Y, const float* tf, const FPrep& pp, int e) {
+template <class B>
+__device__ __forceinline__ void t_hilo(B& Y, const float* tf, const FPrep& pp, int e) {
   const int t = e >> 6, s4 = e & 63;
   const int bi = t >> 4, bj = s4 >> 4;
   const bool keep = bj <= bi;                                      // lower block
@@ -456,7 +457,8 @@ constexpr int kNP = 4;  // prep waves
 // diagonal tile (ti = 0, 2, 5, 9) also yields the squared L2 norms of its 16
 // keys (its diagonal) and, with Q Q^T on the same reads, of its queries: the
 // lane holding [t][t] writes rk[t] and rqs[t] (scale included).
-__device__ __forceinline__ void kq_tile(const FBuf& Y, FPrep& pp, const FusedArgs& a, int ti, f32x4v& kk, f32x4v& qk,
+template <class B>
+__device__ __forceinline__ void kq_tile(const B& Y, FPrep& pp, const FusedArgs& a, int ti, f32x4v& kk, f32x4v& qk,
                                         int r16, int quad) {
   kk = qk = f32x4v{0.f, 0.f, 0.f, 0.f};
   const int mt = lblock_row(ti), m0 = 16 * mt, n0 = 16 * (ti - mt * (mt + 1) / 2);
@@ -481,7 +483,8 @@ __device__ __forceinline__ void kq_tile(const FBuf& Y, FPrep& pp, const FusedArg
 // ... and its L and A entries: row t = m0 + r16, columns s = n0 + 4 quad + 0..3
 // (one 16-byte L write and one 8-byte A write); the decay exponents G_t - G_s
 // are <= 0 for s <= t.
-__device__ __forceinline__ void la_tile(FBuf& Y, const FPrep& pp, int ti, const f32x4v& kk, const f32x4v& qk, int r16,
+template <class B>
+__device__ __forceinline__ void la_tile(B& Y, const FPrep& pp, int ti, const f32x4v& kk, const f32x4v& qk, int r16,
                                         int quad) {
   const int mt = lblock_row(ti), m0 = 16 * mt, n0 = 16 * (ti - mt * (mt + 1) / 2);
   const int t = m0 + r16, s0 = n0 + 4 * quad;
@@ -851,8 +854,28 @@ constexpr int kRecord = kRecT + kRecA + kRecS;
 
 __device__ __forceinline__ int64_t first_slot(const int32_t* cu, int n) { return cu[n] / kC + n; }
 
-__global__ void __launch_bounds__(256) chunk_prep_kernel(FusedArgs a, uint4* ws) {
-  __shared__ FBuf Y;
+// One chunk's buffer: T and A take the place of Q and K, which are read for the
+// last time before either is written, so that three workgroups fit a CU.
+struct __align__(16) PrepBuf {
+  union {
+    struct {
+      uint4 q[kC * 16], k[kC * 16];  // as in FBuf
+    };
+    struct {
+      float t[kC * SF];
+      uint4 aqk[kC * 8];
+    };
+  };
+  union {
+    uint4 p[kC * 16];
+    float l[kC * SF];
+  } tt;
+  float scal[4 * kC];
+  uint32_t gw[2 * kC];
+};
+
+__global__ void __launch_bounds__(256, 3) chunk_prep_kernel(FusedArgs a, uint4* ws) {
+  __shared__ PrepBuf Y;
   __shared__ FPrep pp;
   const int hv = blockIdx.x % a.HV, hk = hv / (a.HV / a.H);
   const int64_t slot = blockIdx.x / a.HV;
@@ -869,10 +892,6 @@ __global__ void __launch_bounds__(256) chunk_prep_kernel(FusedArgs a, uint4* ws)
   fdma_q<0, 4>(Y, a, tok, Lp, hk);
   fdma_k<0, 4>(Y, a, tok, Lp, hk);
   fdma_g<0>(Y, a, tok, Lp, hv);
-  if (tid < 2 * 16 * 4) {  // A's halves in the upper blocks (0, 1) and (2, 3)
-    const int rr = tid >> 2, t = rr < 16 ? rr : 16 + rr, p = t < 16 ? (tid & 3) : 4 + (tid & 3);
-    reinterpret_cast<uint2*>(&Y.aqk[tpos(t, p)])[1] = make_uint2(0, 0);
-  }
   dma_wait();
   lds_barrier();
 
@@ -891,6 +910,10 @@ __global__ void __launch_bounds__(256) chunk_prep_kernel(FusedArgs a, uint4* ws)
     if (w + 4 * i < 10) kq_tile(Y, pp, a, w + 4 * i, kk[i], qk[i], r16, quad);
   lds_barrier();
 
+  if (tid < 2 * 16 * 4) {  // A's halves in the upper blocks (0, 1) and (2, 3)
+    const int rr = tid >> 2, t = rr < 16 ? rr : 16 + rr, p = t < 16 ? (tid & 3) : 4 + (tid & 3);
+    reinterpret_cast<uint2*>(&Y.aqk[tpos(t, p)])[1] = make_uint2(0, 0);
+  }
   if (w == 3) {
     const float eg = expf(pp.G[lane]);
     Y.scal[lane] = eg * pp.rqs[lane];
@@ -903,7 +926,7 @@ __global__ void __launch_bounds__(256) chunk_prep_kernel(FusedArgs a, uint4* ws)
     if (w + 4 * i < 10) la_tile(Y, pp, w + 4 * i, kk[i], qk[i], r16, quad);
   lds_barrier();
 
-  float* tf = Y.vt.t;
+  float* tf = Y.t;
   if (w == 0) inv_diag(Y.tt.l, tf);
   lds_barrier();
   f32x4v y0, y1;
@@ -1102,8 +1125,8 @@ __global__ void __launch_bounds__(CT * 256) chunk_scan_kernel(FusedArgs a, const
 
 // The split form pays while its scan, 4 workgroups a head of 128 columns, runs
 // in one round (one workgroup a CU) and a sequence has a few chunks on average.
-// Two sequences x 32 heads: 123 us against 167; four of 4000 tokens: 417 against
-// 361.  One sequence of 300 tokens: 50 against 60; of 50: 43 against 40.
+// Two sequences x 32 heads: 113 us against 165; four of 4000 tokens: 417 against
+// 361.  One sequence of 300 tokens: 32 against 46; of 50: 43 against 40.
 bool split_form(int64_t total_tokens, int64_t n_seqs, int64_t HV, int64_t V) {
   return n_seqs * HV * (V / 32) <= 256 && total_tokens > 128 * n_seqs &&
          (total_tokens / kC + n_seqs) * HV * kRecord * 16 <= (1LL << 31);   // scratch of at most 2 GiB
