@@ -136,6 +136,22 @@ def test_packed_ragged_prefill_equals_per_prompt_prefill():
         _assert_caches_close([c[r: r + 1] for c in caches], alone)
 
 
+def test_prefill_head_reads_the_row_major_weight():
+    """prepare() makes packed copies for the decode step only: a prefill
+    follows a change of ``lm_head`` made after it, without another prepare."""
+    class Packing(HostOps):
+        @staticmethod
+        def linear(x, w, packed=None, residual=None, defer=False):
+            return HostOps.linear(x, w if packed is None else packed, residual=residual, defer=defer)
+
+    m, ref = _small_model(Packing()), _small_model()
+    prompts = _prompts([5, 70, 1])
+    m.lm_head_packed = m.lm_head.clone()
+    for x in (m, ref):
+        x.lm_head.mul_(-2.0)
+    assert torch.equal(m.prefill(prompts)[0], ref.prefill(prompts)[0])
+
+
 def test_pieced_prefill_equals_whole_prefill():
     """A prompt taken in pieces (each continuing the GDN state, the conv
     window, the ring as left context and the memory through _sequence with a

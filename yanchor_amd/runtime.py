@@ -863,7 +863,7 @@ class Model:
                 src = torch.tensor([off[i] + lens[i] - 1 for i in ends], device=dev)
                 last.index_copy_(0, torch.tensor(ends, device=dev), h.index_select(0, src))
         xn = self.ops.rmsnorm(last, self.final_norm, c.rms_eps)
-        logits = self.ops.linear(xn, self.lm_head, self.lm_head_packed).float()
+        logits = F.linear(xn, self.lm_head).float()
         return logits, tmp.cache_tensors()
 
     def _prefill_piece(self, tmp, tokens, starts, lens):
