@@ -97,6 +97,62 @@ def test_swa_prefill_tiles(gpu, heads, groups, window, lengths, starts, dtype):
     assert ((again.cpu().double() - ref).norm() / ref.norm()).item() < 2e-2
 
 
+def _one_key(dtype, tail):
+    """Queries of 25 lengths and 1024 keys along one dim: score 8 a / sqrt(128)
+    for key 0, 0 for the others, so that those weigh exp(-5.3) .. exp(-7.3) each
+    (tail: exp(-9.5) .. exp(-10.5), subnormal in float16)."""
+    a = torch.linspace(13.5, 15.0, 25) if tail else torch.linspace(7.5, 10.5, 25)
+    q, k = torch.zeros(25, 128, dtype=dtype), torch.zeros(1024, 128, dtype=dtype)
+    q[:, 0], k[0, 0] = a, 8.0
+    p = torch.exp(q[:, :1].double() * -8.0 / 128 ** 0.5)
+    return q, k, p
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_softmax_denominator_keeps_float32(gpu, dtype):
+    """Only key 0 has a value, so a row is value / (1 + 1023 p), and with the sum
+    in float32 it is that to about 2e-6 before its one rounding: all but the
+    values so near a rounding boundary (1 % in float16, whose steps are 2^-11)
+    are the rounded reference.  Sums of rounded p miss it in 16 % of the values."""
+    gen = torch.Generator().manual_seed(1)
+    q, k, p = _one_key(dtype, False)
+    v = (1 + torch.rand(1, 128, generator=gen)).to(dtype)
+    want = v[0].double() / (1 + 1023 * p)
+    # key 0 lies in the first key tile, so the others are weighed against it: in
+    # the ring, 30 keys after the oldest of a piece at position 5000
+    rk, rv = torch.zeros(2, 1, 1, 1024, 128, dtype=dtype)
+    rk[0, 0, (5000 - 1023 + 30) % 1024], rv[0, 0, (5000 - 1023 + 30) % 1024] = k[0], v[0]
+    zero = torch.zeros(25, 1, 128, dtype=dtype, device=gpu)
+    got = layers.swa_prefill(q[:, None].to(gpu), zero, zero, _cu([25], gpu), torch.tensor([5000], device=gpu),
+                             rk.to(gpu), rv.to(gpu), torch.zeros(1, dtype=torch.long, device=gpu)).cpu()[:, 0].double()
+    assert (got != want.to(dtype).double()).double().mean().item() <= 0.02
+
+
+@pytest.mark.parametrize("form", ["window", "memory"])
+def test_subnormal_float16_weights(gpu, form):
+    """One dominant key over 1023 keys whose weights (and their lo parts) are
+    subnormal in float16, a few per cent of the sum.  Bound: the result's own
+    rounding, 2^-11, and that of p to steps of 2^-24 (half a step against 2.6e-5,
+    2^-9.8, of the 4 % they add up to): 2^-10."""
+    gen = torch.Generator().manual_seed(2)
+    q, k, p = _one_key(torch.float16, True)
+    v = (1 + torch.rand(1024, 128, generator=gen)).to(torch.float16)
+    if form == "window":   # query t reads 999 ring slots and the piece up to t
+        rk, rv = torch.zeros(2, 1, 1, 1024, 128, dtype=torch.float16)
+        rk[0, 0, 0], rv[0, 0, :999] = k[0], v[:999]
+        got = layers.swa_prefill(q[:, None].to(gpu), k[999:, None].to(gpu), v[999:, None].to(gpu), _cu([25], gpu),
+                                 torch.tensor([999], device=gpu), rk.to(gpu), rv.to(gpu),
+                                 torch.zeros(1, dtype=torch.long, device=gpu)).cpu()[:, 0].double()
+        tail = v[1:999].double().sum(0) + v[999:].double().cumsum(0)
+        want = (v[0].double() + p * tail) / (1 + p * (999 + torch.arange(25)[:, None]))
+    else:                  # the sink's logit is 0 as well
+        refs = torch.arange(1024, dtype=torch.int32).view(1, 1, 1, 1024).to(gpu)
+        got = im.indexed_gqa(q.view(1, 1, 25, 1, 128).to(gpu), k.view(1, 1024, 1, 128).to(gpu),
+                             v.view(1, 1024, 1, 128).to(gpu), refs).cpu().view(25, 128).double()
+        want = (v[0].double() + p * v[1:].double().sum(0)) / (1 + p * 1024)
+    assert ((got - want).norm() / want.norm()).item() <= 2 ** -10
+
+
 def _memory_state(gen, b, g, cap, chunk, counts, base, dtype, odd):
     """A memory state with committed slots in no particular order, ``counts``
     pending tokens a row and positions below ``base``.  odd: tied scores, empty

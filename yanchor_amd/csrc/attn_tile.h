@@ -12,8 +12,8 @@
 // so neither P nor O leaves registers.
 //
 // What bounds it: the softmax's vector work (a fma, a quarter-rate exp2, half a
-// conversion and half a dot product a score, and a rescaling of the
-// accumulators a tile) and the MFMAs take 1300 and 1024 cycles of a SIMD a
+// conversion and an addition a score, and a rescaling of the accumulators a
+// tile) and the MFMAs take 1300 and 1024 cycles of a SIMD a
 // tile; two waves a SIMD overlap them only in part, the rest is waits on LDS
 // and on the tile's barrier.  Hence: key tiles by direct global-to-LDS copies,
 // double buffered, one barrier a tile; 16-byte pieces swizzled so that the
@@ -22,10 +22,9 @@
 // product between the MFMAs of the step before; a raised wave priority around
 // the MFMAs, so that they run under the other wave's vector work; no mask code on
 // tiles where every key is live.  Six waves a workgroup (three a SIMD, 168
-// registers) take 1.4 times as long even with the addresses re-formed a tile.  The denominator sums the
-// rounded P that the value product sees (two at a time, v_dot2), so the
-// rounding of a dominant probability cancels in the quotient.  (A running
-// maximum that lags the scores by up to 2^8 and leaves out most rescalings was
+// registers) take 1.4 times as long even with the addresses re-formed a tile.  The
+// denominator sums P in float32, before the rounding that the value product
+// sees.  (A running maximum that lags the scores by up to 2^8 and leaves out most rescalings was
 // 10 % faster and 2 % further from float64: a row's largest probability is
 // exact only while the maximum is.)
 #pragma once
@@ -58,10 +57,6 @@ struct Mfma<YH_BF16> {
   static __device__ __forceinline__ uint32_t round2(float x, float y) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){x, y}, bf16x2_t));
   }
-  static __device__ __forceinline__ float sum2(uint32_t p, float c) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, p), __builtin_bit_cast(bf16x2_t, 0x3f803f80u), c,
-                                           false);
-  }
   static __device__ __forceinline__ uint16_t round(float x) { return f32_to_bf16(x); }
   static __device__ __forceinline__ float widen(uint16_t h) { return bf16_to_f32(h); }
 };
@@ -73,9 +68,6 @@ struct Mfma<YH_F16> {
   }
   static __device__ __forceinline__ uint32_t round2(float x, float y) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){x, y}, f16x2_t));
-  }
-  static __device__ __forceinline__ float sum2(uint32_t p, float c) {
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, p), __builtin_bit_cast(f16x2_t, 0x3c003c00u), c, false);
   }
   static __device__ __forceinline__ uint16_t round(float x) { return f32_to_f16(x); }
   static __device__ __forceinline__ float widen(uint16_t h) { return f16_to_f32(h); }
@@ -237,11 +229,9 @@ struct State {
       const float p1 = __builtin_amdgcn_exp2f(fmaf(c[ks >> 1][8 * (ks & 1) + 2 * e + 1], k2, -base));
       const uint32_t h = M::round2(p0, p1);
       ph[ks & 1][e] = h;
-      den = M::sum2(h, den);
-      if constexpr (HILO) {
+      den += p0 + p1;
+      if constexpr (HILO)
         pl[ks & 1][e] = M::round2(p0 - M::widen(static_cast<uint16_t>(h)), p1 - M::widen(static_cast<uint16_t>(h >> 16)));
-        den = M::sum2(pl[ks & 1][e], den);
-      }
     };
     constexpr int kAhead = 3;   // V operands in flight
     vec vf[kAhead];
