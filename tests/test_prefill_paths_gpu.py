@@ -97,6 +97,32 @@ def test_swa_prefill_tiles(gpu, heads, groups, window, lengths, starts, dtype):
     assert ((again.cpu().double() - ref).norm() / ref.norm()).item() < 2e-2
 
 
+@pytest.mark.parametrize("heads,groups,tt", [(32, 8, 16), (2, 2, 64), (16, 2, 8)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_swa_prefill_unseen_values(gpu, heads, groups, tt, bad):
+    """A value that is not finite reaches no token before the tile of ``tt``
+    tokens it lies in and none after the last tile with a token that sees it,
+    whatever shares the workgroup: those rows are bit for bit what they are
+    without it."""
+    gen = torch.Generator().manual_seed(9)
+    n, window, bf = 6 * tt + 200, 64, torch.bfloat16
+    q, k, v = (torch.randn(n, h, 128, generator=gen).to(bf) for h in (heads, groups, groups))
+    ring = torch.randn(1, groups, window, 128, generator=gen).to(bf)
+
+    def run(x):
+        return layers.swa_prefill(q.to(gpu), k.to(gpu), x.to(gpu), _cu([n], gpu), torch.tensor([70], device=gpu),
+                                  ring.to(gpu), ring.to(gpu), torch.zeros(1, dtype=torch.long, device=gpu)).cpu()
+    clean = run(v)
+    for at in (0, tt, 2 * tt + 1, 3 * tt, 4 * tt - 1):
+        x = v.clone()
+        x[at] = bad
+        got = run(x)
+        first, last = at // tt * tt, (at + window - 1) // tt * tt + tt
+        assert not torch.isfinite(got[at].float()).any()
+        assert torch.equal(got[:first], clean[:first]), at
+        assert torch.equal(got[last:], clean[last:]), at
+
+
 def _one_key(dtype, tail):
     """Queries of 25 lengths and 1024 keys along one dim: score 8 a / sqrt(128)
     for key 0, 0 for the others, so that those weigh exp(-5.3) .. exp(-7.3) each

@@ -153,7 +153,7 @@ __global__ void __launch_bounds__(NW * 64, 2) indexed_gqa_kernel(IdxArgs a) {
       if (last && left > 1) live_after = load_queries(nb + 1);   // the scores are the last use of this block's
       if (have != ~0ull)
         st.mask(c, [&](int key, int half) { return (have >> (key + 4 * half)) & 1; });
-      st.template step<true>(c, vtile[buf], k2);
+      st.template step<true, false>(c, vtile[buf], k2);
     } else if (last && left > 1) {
       live_after = load_queries(nb + 1);
     }

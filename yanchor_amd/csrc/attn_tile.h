@@ -190,9 +190,11 @@ struct State {
       for (int i = 0; i < 16; ++i) c[kt][i] = live(kt * 32 + 8 * (i >> 2) + (i & 3), half) ? c[kt][i] : -INFINITY;
   }
   // The softmax of a tile's scores c and its value product.  HILO: P enters the
-  // product as a hi + lo pair.  k2 = scale * log2(e).
-  template <bool HILO>
-  __device__ __forceinline__ void step(const f32x16 (&c)[2], const Rows& v, float k2) {
+  // product as a hi + lo pair.  k2 = scale * log2(e).  EDGE: keep (wave-uniform)
+  // has a bit for each key of the tile; the others' values count as zeros, since
+  // a weight of 0 does not take out a value that is not finite.
+  template <bool HILO, bool EDGE>
+  __device__ __forceinline__ void step(const f32x16 (&c)[2], const Rows& v, float k2, uint64_t keep = ~0ull) {
     using M = Mfma<DT>;
     using vec = typename M::vec;
     const int lane = lane_id(), half = lane >> 5;
@@ -233,6 +235,18 @@ struct State {
       if constexpr (HILO)
         pl[ks & 1][e] = M::round2(p0 - M::widen(static_cast<uint16_t>(h)), p1 - M::widen(static_cast<uint16_t>(h >> 16)));
     };
+    // word e of a V operand of step ks holds keys 16 ks + 8 (e / 2) + 4 half + 2 (e % 2) and the next
+    uint32_t kept[4];
+    auto find_kept = [&](int ks) {
+      const uint32_t live = static_cast<uint32_t>(keep >> (32 * (ks >> 1))) >> (4 * half);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int bit = 16 * (ks & 1) + 8 * (e >> 1) + 2 * (e & 1);
+        const uint32_t even = static_cast<int32_t>(live << (31 - bit)) >> 31;
+        const uint32_t odd = static_cast<int32_t>(live << (30 - bit)) >> 31;
+        kept[e] = (even & 0xffffu) | (odd & 0xffff0000u);
+      }
+    };
     constexpr int kAhead = 3;   // V operands in flight
     vec vf[kAhead];
 #pragma unroll
@@ -246,6 +260,12 @@ struct State {
       const int d = n & 3, ks = n >> 2;
       const uint32_t* h = ph[ks & 1];
       if (ks == 0) acc[d] *= alpha;
+      if constexpr (EDGE) {
+        if (d == 0) find_kept(ks);
+        const uint4 x = __builtin_bit_cast(uint4, vf[n % kAhead]);
+        vf[n % kAhead] =
+            __builtin_bit_cast(vec, make_uint4(x.x & kept[0], x.y & kept[1], x.z & kept[2], x.w & kept[3]));
+      }
       acc[d] = M::run(vf[n % kAhead], __builtin_bit_cast(vec, make_uint4(h[0], h[1], h[2], h[3])), acc[d]);
       if constexpr (HILO) {
         const uint32_t* l = pl[ks & 1];

@@ -26,6 +26,8 @@
 // R query heads of a KV group.  A workgroup of NW waves takes NW / 2 tiles that
 // follow each other in the list, two waves each; the tiles of one piece share
 // their key tiles (attn_tile.h).
+#include <type_traits>
+
 #include "attn_tile.h"
 
 namespace yh {
@@ -311,23 +313,43 @@ __global__ void __launch_bounds__(NW * 64, 2) swa_prefill_kernel(SwaArgs a) {
     const int wlo = nctx + wtok, whi = nctx + min(wtok + wspan, len) - 1;
     const bool in = active && mine >= i0 && mine < i1 && wtok < len;
     auto sees = [&](int j0) { return in && j0 <= whi && j0 + attn::kTile - 1 > wlo - W; };
+    // the keys of such a tile that any of them sees: the others are a later
+    // tile's, or the oldest of an earlier one
+    auto seen = [&](int j0) {
+      const int lo = max(wlo - W + 1 - j0, 0), hi = min(whi - j0, attn::kTile - 1);
+      return (~0ull << (lo & 63)) & (~0ull >> ((attn::kTile - 1 - hi) & 63));
+    };
     load(ktile[0], j_lo, a.k, a.k_ts, a.ring_k);
     load(vtile[0], j_lo, a.v, a.v_ts, a.ring_v);
-    int buf = 0;
-    for (int j0 = j_lo; j0 <= j_hi; j0 += attn::kTile, buf ^= 1) {
+    int buf = 0, j0 = j_lo;
+    auto tile = [&](auto edge, uint64_t keep) {
       attn::copy_wait();      // this wave's part of the tile has arrived
       attn::tile_barrier();   // everyone's has, and the other buffers are consumed
       load(ktile[buf ^ 1], j0 + attn::kTile, a.k, a.k_ts, a.ring_k);
       load(vtile[buf ^ 1], j0 + attn::kTile, a.v, a.v_ts, a.ring_v);
-      if (!sees(j0)) continue;
-      attn::f32x16 c[2];
-      st.scores(ktile[buf], c);
-      if (j0 + attn::kTile - 1 > wlo || j0 <= whi - W)
-        st.mask(c, [&](int key, int half) {
-          const int j = j0 + key + 4 * half;
-          return j <= self && j > self - W;
-        });
-      st.template step<false>(c, vtile[buf], k2);
+      if (sees(j0)) {
+        attn::f32x16 c[2];
+        st.scores(ktile[buf], c);
+        if constexpr (edge.value)
+          st.mask(c, [&](int key, int half) {
+            const int j = j0 + key + 4 * half;
+            return j <= self && j > self - W;
+          });
+        st.template step<false, edge.value>(c, vtile[buf], k2, keep);
+      }
+      j0 += attn::kTile;
+      buf ^= 1;
+    };
+    // Every key of an inner tile is live for every query of the wave.  The two
+    // kinds take a loop each (the waves of a workgroup change over on their own:
+    // both pass one barrier a tile): as branches of one loop they spill 97
+    // registers, and a branch at each value operand costs 9 % of the kernel.
+    auto inner = [&]() { return j0 + attn::kTile - 1 <= wlo && j0 > whi - W; };
+    while (j0 <= j_hi) {
+#pragma unroll 1
+      while (j0 <= j_hi && inner()) tile(std::false_type{}, ~0ull);
+#pragma unroll 1
+      while (j0 <= j_hi && !inner()) tile(std::true_type{}, seen(j0));
     }
     attn::copy_wait();
     attn::tile_barrier();     // the buffers are consumed
