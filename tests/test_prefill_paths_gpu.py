@@ -123,6 +123,37 @@ def test_swa_prefill_unseen_values(gpu, heads, groups, tt, bad):
         assert torch.equal(got[last:], clean[last:]), at
 
 
+def test_swa_prefill_scattered_tiles(gpu):
+    """A caller's tile list whose neighbours lie far apart costs about what the
+    sorted list does (each tile its own window, at most twice the copies): the
+    keys between two tiles of a piece are not walked.  Walking them took 8 times
+    as long here; the bound is 5."""
+    n, window, bf = 16000, 64, torch.bfloat16
+    q, k, v = (torch.randn(n, h, 128, device=gpu).to(bf) for h in (32, 8, 8))
+    ring = torch.zeros(1, 8, window, 128, dtype=bf, device=gpu)
+    at = torch.zeros(1, dtype=torch.long, device=gpu)
+    tiles = layers.prefill_tiles([n], 16, "cpu")
+    mixed = tiles[torch.randperm(len(tiles), generator=torch.Generator().manual_seed(0))]
+    launch, times, outs = _native.call, [], []
+
+    def timed(name, *args):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        launch(name, *args)
+        b.record()
+        b.synchronize()
+        times.append(a.elapsed_time(b))
+    try:
+        _native.call = timed
+        for _ in range(5):
+            for order in (tiles, mixed):
+                outs.append(layers.swa_prefill(q, k, v, _cu([n], gpu), at, ring, ring, at, tiles=order))
+    finally:
+        _native.call = launch
+    assert torch.equal(outs[-1], outs[-2]) or (outs[-1].float() - outs[-2].float()).abs().max() < 0.05
+    assert min(times[1::2]) <= 5 * min(times[::2]), times
+
+
 def _one_key(dtype, tail):
     """Queries of 25 lengths and 1024 keys along one dim: score 8 a / sqrt(128)
     for key 0, 0 for the others, so that those weigh exp(-5.3) .. exp(-7.3) each

@@ -265,12 +265,14 @@ __global__ void __launch_bounds__(NW * 64, 2) swa_prefill_kernel(SwaArgs a) {
   const float k2 = a.scale * 1.4426950408889634f;
 
   for (int i0 = 0; i0 < count;) {
-    // the tiles i0 .. i1 - 1 of one piece: the union of their key ranges
+    // the tiles i0 .. i1 - 1 of one piece whose windows meet: the union of their key ranges
     const int pr = list[2 * i0];
     int lo = list[2 * i0 + 1], hi = lo, i1 = i0 + 1;
     for (; i1 < count && list[2 * i1] == pr; ++i1) {
-      lo = min(lo, list[2 * i1 + 1]);
-      hi = max(hi, list[2 * i1 + 1]);
+      const int t = list[2 * i1 + 1];
+      if (max(hi, t) - min(lo, t) > W) break;   // nothing to share, and the keys between would be copied for nobody
+      lo = min(lo, t);
+      hi = max(hi, t);
     }
     const int64_t ps = a.cu[pr];
     const int plen = a.cu[pr + 1] - a.cu[pr];
