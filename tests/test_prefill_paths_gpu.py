@@ -305,3 +305,37 @@ def test_gdn_few_sequences(gpu, lengths, h, hv, v, h0, gates):
     many_o, many_st = run(copies)
     assert torch.equal(o, many_o[:, :n]) and torch.equal(st, many_st[: len(lengths)])
     assert torch.equal(o, many_o[:, -n:]) and torch.equal(st, many_st[-len(lengths):])
+
+
+@pytest.mark.parametrize("n,length,hv", [(64, 200, 1), (32, 130, 1), (8, 140, 4), (2, 150, 32), (1, 129, 32)])
+def test_gdn_few_sequences_time(gpu, n, length, hv):
+    """At the edge of its rule (short sequences, many of few heads) the split form
+    is no slower than the one launch it stands for (best of 40, 4 % for the
+    clock)."""
+    total = n * length
+    q, k, v = (torch.randn(total, hv, 128, device=gpu).to(torch.bfloat16) for _ in range(3))
+    g, beta = -0.1 * torch.rand(total, hv, device=gpu), torch.rand(total, hv, device=gpu)
+    cu, o = _cu([length] * n, gpu), torch.empty_like(v)
+    state = torch.empty(n, hv, 128, 128, device=gpu)
+    need = _native.lib().yh_gdn_chunk_workspace_bytes(total, n, hv, 128)
+    ws = torch.empty(need, dtype=torch.uint8, device=gpu)
+    assert need > 0
+
+    def best(scratch, size):
+        times = []
+        for _ in range(40):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(5):
+                _native.call("yh_gdn_chunk_varlen", q.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(),
+                             beta.data_ptr(), None, state.data_ptr(), o.data_ptr(), cu.data_ptr(), None, n, total, hv,
+                             hv, 128, 128, 128 ** -0.5, 1, _native.BF16, _native.F32, _native.F32, scratch, size,
+                             _native.stream_of(q))
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+    best(ws.data_ptr(), need)
+    split, one = best(ws.data_ptr(), need), best(None, 0)
+    print(n, length, hv, 'us:', split * 200, one * 200, flush=True)
+    assert split <= 1.04 * one

@@ -879,8 +879,12 @@ __global__ void __launch_bounds__(256, 3) chunk_prep_kernel(FusedArgs a, uint4* 
   __shared__ FPrep pp;
   const int hv = blockIdx.x % a.HV, hk = hv / (a.HV / a.H);
   const int64_t slot = blockIdx.x / a.HV;
-  int n = a.n_seqs - 1;
-  while (n > 0 && first_slot(a.cu, n) > slot) --n;
+  int n = 0;
+  for (int hi = a.n_seqs - 1; n < hi;) {   // the last sequence whose slots start at or before this one
+    const int mid = (n + hi + 1) >> 1;
+    if (first_slot(a.cu, mid) <= slot) n = mid;
+    else hi = mid - 1;
+  }
   const int j = static_cast<int>(slot - first_slot(a.cu, n));
   const int seqlen = a.cu[n + 1] - a.cu[n];
   if (j * kC >= seqlen) return;   // a slot without a chunk

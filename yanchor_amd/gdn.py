@@ -162,13 +162,14 @@ def chunk_gated_delta_rule(query, key, value, g=None, beta=None, scale=None, ini
     if _chunk_kernel_fits(q, v) and not force_recurrent:
         h0 = None if initial_state is None else initial_state.contiguous()
         state = torch.empty(n, hv, kd, vd, device=dev, dtype=torch.float32)
-        order = None
-        if lengths is not None and n > 1:  # longest sequences first balances the grid
-            order = torch.tensor(sorted(range(n), key=lambda i: -int(lengths[i])), dtype=torch.int32,
-                                 device=dev)
         # scratch for the few-sequences form; none otherwise
         need = N.lib().yh_gdn_chunk_workspace_bytes(total, n, hv, vd)
         ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+        order = None
+        # longest sequences first balances the grid, which the few-sequences form runs in one round
+        if lengths is not None and n > 1 and ws is None:
+            order = torch.tensor(sorted(range(n), key=lambda i: -int(lengths[i])), dtype=torch.int32,
+                                 device=dev)
         N.call("yh_gdn_chunk_varlen", q.data_ptr(), k.data_ptr(), v.data_ptr(), g_.data_ptr(), be.data_ptr(),
                N.ptr(h0), state.data_ptr(), o.data_ptr(), cu.data_ptr(), N.ptr(order), n, total, h, hv, kd, vd, sc,
                int(bool(use_qk_l2norm_in_kernel)), N.code(q), N.code(g_), N.code(be), N.ptr(ws), need, N.stream_of(q))
