@@ -307,6 +307,16 @@ def test_gdn_few_sequences(gpu, lengths, h, hv, v, h0, gates):
     assert torch.equal(o, many_o[:, -n:]) and torch.equal(st, many_st[-len(lengths):])
 
 
+@pytest.mark.parametrize("lens", [[300], [300, 200], [10] * 9])
+def test_gdn_lengths_of_every_sequence(gpu, lens):
+    """A ``lengths`` that misses a sequence is refused whichever form runs."""
+    total, hv = sum(lens), 32
+    x = torch.zeros(1, total, hv, 128, dtype=torch.bfloat16, device=gpu)
+    g = torch.zeros(1, total, hv, device=gpu)
+    with pytest.raises(IndexError):
+        gdn.chunk_gated_delta_rule(x, x, x, g=g, beta=g, cu_seqlens=_cu(lens, gpu), lengths=lens[:-1])
+
+
 @pytest.mark.parametrize("n,length,hv", [(64, 200, 1), (32, 130, 1), (8, 140, 4), (2, 150, 32), (1, 129, 32)])
 def test_gdn_few_sequences_time(gpu, n, length, hv):
     """At the edge of its rule (short sequences, many of few heads) the split form

@@ -160,6 +160,8 @@ def chunk_gated_delta_rule(query, key, value, g=None, beta=None, scale=None, ini
     o = torch.empty(1, total, hv, vd, device=dev, dtype=value.dtype)
     sc = float(kd ** -0.5 if scale is None else scale)
     if _chunk_kernel_fits(q, v) and not force_recurrent:
+        if lengths is not None and len(lengths) < n:
+            raise IndexError("lengths must hold one length per sequence")
         h0 = None if initial_state is None else initial_state.contiguous()
         state = torch.empty(n, hv, kd, vd, device=dev, dtype=torch.float32)
         # scratch for the few-sequences form; none otherwise
