@@ -307,6 +307,27 @@ def test_gdn_few_sequences(gpu, lengths, h, hv, v, h0, gates):
     assert torch.equal(o, many_o[:, -n:]) and torch.equal(st, many_st[-len(lengths):])
 
 
+def test_gdn_no_room_for_scratch(gpu, monkeypatch):
+    """The few-sequences form's scratch is not a condition of the call: without
+    room for it the call gives the same bits."""
+    x = torch.randn(1, 700, 4, 128, device=gpu).to(torch.bfloat16)
+    g = -torch.rand(1, 700, 4, device=gpu)
+    args = dict(g=g, beta=-g, output_final_state=True, cu_seqlens=_cu([700], gpu), use_qk_l2norm_in_kernel=True)
+    want = gdn.chunk_gated_delta_rule(x, x, x, **args)
+    need = _native.lib().yh_gdn_chunk_workspace_bytes(700, 1, 4, 128)
+    empty, refused = torch.empty, []
+
+    def no_scratch(*size, **kw):
+        if size == (need,):
+            refused.append(size)
+            raise torch.OutOfMemoryError("no room")
+        return empty(*size, **kw)
+    monkeypatch.setattr(torch, "empty", no_scratch)
+    got = gdn.chunk_gated_delta_rule(x, x, x, **args)
+    monkeypatch.undo()
+    assert refused and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 @pytest.mark.parametrize("lens", [[300], [300, 200], [10] * 9])
 def test_gdn_lengths_of_every_sequence(gpu, lens):
     """A ``lengths`` that misses a sequence is refused whichever form runs."""

@@ -120,8 +120,9 @@ def chunk_gated_delta_rule(query, key, value, g=None, beta=None, scale=None, ini
     ``force_recurrent=True``, run the token-recurrent kernel over each
     sequence.  ``lengths`` (host ints, one per sequence) lets the chunk
     kernel start the longest sequences first.  Scratch memory, which only
-    calls of few sequences need, belongs to the call, so concurrent calls on
-    different streams are independent.
+    calls of few sequences use (25.6 KB per 64 tokens and value head, at most
+    2 GiB) and do without where there is no room for it, belongs to the call,
+    so concurrent calls on different streams are independent.
     """
     if g is None or beta is None:
         raise ValueError("chunk_gated_delta_rule needs g and beta")
@@ -164,9 +165,15 @@ def chunk_gated_delta_rule(query, key, value, g=None, beta=None, scale=None, ini
             raise IndexError("lengths must hold one length per sequence")
         h0 = None if initial_state is None else initial_state.contiguous()
         state = torch.empty(n, hv, kd, vd, device=dev, dtype=torch.float32)
-        # scratch for the few-sequences form; none otherwise
+        # scratch for the few-sequences form; none otherwise, and none (the one-launch
+        # form, the same bits) where the device has no room for it
         need = N.lib().yh_gdn_chunk_workspace_bytes(total, n, hv, vd)
-        ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+        ws = None
+        if need:
+            try:
+                ws = torch.empty(need, dtype=torch.uint8, device=dev)
+            except torch.OutOfMemoryError:
+                need = 0
         order = None
         # longest sequences first balances the grid, which the few-sequences form runs in one round
         if lengths is not None and n > 1 and ws is None:
