@@ -711,22 +711,26 @@ int launch_read_r(int R, const ReadArgs& a, hipStream_t st) {
       // Few memories leave CUs idle while two waves walk a memory's blocks one
       // after the other: up to one memory a CU takes as many waves as a CU
       // holds (window ring) or as its 16 blocks feed (256 slots), up to three a
-      // CU four waves.  1024-slot ring and 256-slot memory, 8 memories a row,
-      // us with two waves -> with these: 1 row 68 and 20 -> 24 and 10, 32 rows
-      // 69 and 21 -> 30 and 12, 64 rows 78 and 24 -> 51 and 17, 96 rows 91 and 26
-      // -> 76 and 24; 128 rows' memory 29 -> 33.  A memory of a few blocks has
-      // nothing to share out.
+      // CU four waves (16-bit).  1024-slot ring and 256-slot memory, 8 memories a
+      // row, us with two waves -> with these: 1 row 68 and 20 -> 24 and 10 (272
+      // slots 22 -> 11, 512 36 -> 15), 32 rows 69 and 21 -> 30 and 12, 64 rows 78
+      // and 24 -> 51 and 17, 96 rows 91 and 26 -> 76 and 24; 128 rows' memory 29 ->
+      // 33.  float32 keeps two past one memory a CU: 264 memories of 256 slots 24
+      // us, with four 26; 400 26 and 29.  A memory of a few blocks has nothing to
+      // share out.  (The order of a row's sums goes with the number of waves, so
+      // its last bits may change where the batch crosses one of these lines.)
       constexpr int kMany = DT == YH_F32 ? 8 : 12;
+      constexpr int64_t kFour = DT == YH_F32 ? 256 : 768;   // memories that four waves still pay for
       const int64_t memories = static_cast<int64_t>(a.B) * a.G;
-      const int w = a.KC < 64 || memories > 768 ? 2 : memories > 256 ? 4 : a.KC > 256 ? kMany : 6;
+      const int w = a.KC < 64 || memories > kFour ? 2 : memories > 256 ? 4 : a.KC > 256 ? kMany : 6;
       if (w == kMany)
         hipLaunchKernelGGL((anchor_read_kernel<DT, D, 4, SINK, kR4BS, false, kMany>), grid, dim3(kMany * 64), 0, st, a);
       else if (w == 6)
         hipLaunchKernelGGL((anchor_read_kernel<DT, D, 4, SINK, kR4BS, false, 6>), grid, dim3(6 * 64), 0, st, a);
-      else if (w == 4)
-        hipLaunchKernelGGL((anchor_read_kernel<DT, D, 4, SINK, kR4BS, false, 4>), grid, dim3(4 * 64), 0, st, a);
-      else
+      else if (w == 2)
         hipLaunchKernelGGL((anchor_read_kernel<DT, D, 4, SINK, kR4BS, false>), grid, b4, 0, st, a);
+      else if constexpr (DT != YH_F32)
+        hipLaunchKernelGGL((anchor_read_kernel<DT, D, 4, SINK, kR4BS, false, 4>), grid, dim3(4 * 64), 0, st, a);
       break;
     }
     default: set_error("anchor_read: heads per group must be 1, 2 or 4 (got %d)", R); return YH_ERR_INVALID;
