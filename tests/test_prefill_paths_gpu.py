@@ -277,6 +277,29 @@ def test_memory_sequence_segments(gpu, cap, chunk, length, heads, groups, odd):
     assert torch.equal(again, got[valid.to(gpu)])
 
 
+@pytest.mark.parametrize("offsets", [[0, 8, 10], [0, 5, 9], [0, 5], [1, 5, 10], [0, 5, 11]])
+def test_memory_sequence_packed_offsets(gpu, offsets):
+    """Offsets that are not those of ``lengths`` are refused before anything is
+    written; offsets on the host give what those on the device give."""
+    gen = torch.Generator().manual_seed(4)
+    dt, lens = torch.bfloat16, [5, 5]
+    st = _memory_state(gen, 2, 2, 16, 4, [0, 3], 40, dt, False)
+    toks = [torch.randn(10, h, 128, generator=gen).to(dt).to(gpu) for h in (4, 2, 2)] + \
+        [torch.randn(10, 2, generator=gen).to(gpu)]
+    state = _clone(st, gpu)
+    with pytest.raises(ValueError, match="offsets"):
+        im.sequence_packed(*toks, torch.tensor(offsets, dtype=torch.int32, device=gpu), lens, 4, state)
+    for f in fields(st):
+        assert torch.equal(getattr(state, f.name).cpu(), getattr(st, f.name)), f.name
+    outs, states = [], []
+    for cu in (_cu(lens, gpu), _cu(lens, "cpu")):
+        states.append(_clone(st, gpu))
+        outs.append(im.sequence_packed(*toks, cu, lens, 4, states[-1]))
+    for o, s in zip(outs[1:], states[1:]):
+        assert torch.equal(o, outs[0])
+        assert all(torch.equal(getattr(s, f.name), getattr(states[0], f.name)) for f in fields(st))
+
+
 @pytest.mark.parametrize("lengths,h,hv,v,h0,gates", [
     ([3001], 4, 4, 128, True, torch.float32),        # one tile a workgroup, a ragged last chunk
     ([129, 0, 64, 700], 2, 8, 128, False, torch.bfloat16),   # an empty sequence, slots between chunks, GQA

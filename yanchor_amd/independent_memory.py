@@ -16,6 +16,7 @@ from __future__ import annotations
 import ctypes
 import math
 from dataclasses import dataclass, fields
+from itertools import accumulate
 
 import torch
 
@@ -297,8 +298,18 @@ def sequence(query, key, value, scores, valid, chunk, state: IndependentMemorySt
 def sequence_packed(query, key, value, scores, cu_seqlens, lengths, chunk, state: IndependentMemoryState):
     """``sequence`` over ragged rows packed without padding: row r holds
     tokens [cu_seqlens[r], cu_seqlens[r + 1]) of query ``[N, H, D]``, key /
-    value ``[N, G, D]`` and scores ``[N, G]`` (``lengths``: the same lengths on
-    the host, each >= 1).  Returns the read ``[N, H, D]``."""
+    value ``[N, G, D]`` and scores ``[N, G]``.  ``lengths``: the rows' lengths on
+    the host, each >= 1; ``cu_seqlens`` must be their offsets (on the device:
+    compared in a copy that waits for the stream).  Returns the read
+    ``[N, H, D]``."""
+    lengths = [int(x) for x in lengths]
+    if cu_seqlens.tolist() != [0, *accumulate(lengths)]:
+        raise ValueError("cu_seqlens must be the offsets of lengths")
+    return _sequence_packed(query, key, value, scores, cu_seqlens.to(query.device), lengths, chunk, state)
+
+
+def _sequence_packed(query, key, value, scores, cu_seqlens, lengths, chunk, state):
+    """``sequence_packed`` of offsets known to be those of ``lengths``."""
     nb, g, cap, pc, d = _check_state(state)
     n, h = query.shape[:2]
     if query.shape != (n, h, d) or key.shape != (n, g, d) or value.shape != key.shape or scores.shape != (n, g):

@@ -288,8 +288,9 @@ class HipOps:
         return _token_by_token_sequence(self, q, key, value, scores, valid, chunk, state)
 
     def memory_sequence_packed(self, q, key, value, scores, cu, lens, chunk, state):
-        """The same over packed rows of the given lengths (>= 1), 16-bit."""
-        return self.mem.sequence_packed(q, key, value, scores, cu, lens, chunk, state)
+        """The same over packed rows of the given lengths (>= 1) and their
+        offsets cu, 16-bit."""
+        return self.mem._sequence_packed(q, key, value, scores, cu, lens, chunk, state)
 
     def sample(self, logits, attempt_ids, steps, seen, *, seed, temperature, top_k, top_p, penalty,
                backend="triton_top20"):
