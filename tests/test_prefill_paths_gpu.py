@@ -277,6 +277,34 @@ def test_memory_sequence_segments(gpu, cap, chunk, length, heads, groups, odd):
     assert torch.equal(again, got[valid.to(gpu)])
 
 
+@pytest.mark.parametrize("case", ["float32", "heads of 64", "5 heads on 2 groups", "no tokens", "unaligned keys"])
+@pytest.mark.parametrize("packed", [False, True])
+def test_memory_sequence_refusals_leave_the_state(gpu, case, packed):
+    """What the read or the state rewrite cannot take is refused before the scan
+    rewrites the state's scores and positions."""
+    gen = torch.Generator().manual_seed(6)
+    dt, d = torch.float32 if case == "float32" else torch.bfloat16, 64 if case == "heads of 64" else 128
+    h, n = 5 if case[0] == "5" else 4, 0 if case == "no tokens" else 6
+    if packed and n == 0:
+        pytest.skip("packed rows hold at least one token")
+    state = im.IndependentMemoryState.empty(1, 2, 16, 4, d, gpu, dt)
+    state.scores.copy_(torch.randn(state.scores.shape, generator=gen))
+    state.positions.copy_(torch.randint(0, 50, state.positions.shape, generator=gen))
+    state.total.fill_(60)
+    if case == "unaligned keys":
+        state.keys = torch.zeros(state.keys.numel() + 1, dtype=dt, device=gpu)[1:].view(state.keys.shape)
+    before = _clone(state, "cpu")
+    toks = [torch.randn(1, n, x, d, generator=gen).to(dt).to(gpu) for x in (h, 2, 2)] + \
+        [torch.randn(1, n, 2, generator=gen).to(gpu)]
+    with pytest.raises(ValueError):
+        if packed:
+            im.sequence_packed(*[x[0] for x in toks], _cu([n], gpu), [n], 4, state)
+        else:
+            im.sequence(*toks, None, 4, state)
+    for f in fields(state):
+        assert torch.equal(getattr(state, f.name).cpu(), getattr(before, f.name)), f.name
+
+
 @pytest.mark.parametrize("offsets", [[0, 8, 10], [0, 5, 9], [0, 5], [1, 5, 10], [0, 5, 11]])
 def test_memory_sequence_packed_offsets(gpu, offsets):
     """Offsets that are not those of ``lengths`` are refused before anything is

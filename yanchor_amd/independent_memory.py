@@ -342,9 +342,17 @@ def _token_rows(x):
 
 def _sequence_tokens(query, key, value, scores, counts, bases, order, length, c, state, out):
     """The prefix Top-K scan, the read and the state rewrite on tokens in
-    place (yh_anchor_tokens_*): query [N, H, D], key / value [N, G, D]."""
+    place (yh_anchor_tokens_*): query [N, H, D], key / value [N, G, D].  The
+    scan rewrites the state's scores, so what the read or the rewrite after it
+    would refuse is refused before."""
     b, g, cap, d = state.keys.shape
     pc, h, dev = state.pending_keys.shape[2], query.shape[1], query.device
+    if query.dtype not in (torch.bfloat16, torch.float16) or d != 128 or h % g:
+        raise ValueError("the prefill read takes bf16 / fp16 heads of 128 and a multiple of the memory's groups")
+    if b and not length:
+        raise ValueError("a prefill needs at least one token")
+    if any(x.data_ptr() % 16 for x in (state.keys, state.values, state.pending_keys, state.pending_values)):
+        raise ValueError("memory key/value tensors must be 16-byte aligned")
     blocks = -(-length // c) + 1                  # ceil((L + C) / C) blocks of C positions
     block_refs = torch.empty(b, blocks, g, cap, device=dev, dtype=torch.int32)
     final_refs = torch.empty(b, g, cap, device=dev, dtype=torch.int32)
