@@ -752,8 +752,8 @@ int yh_linear_reduce(const float* part, void* out, int64_t out_stride, int64_t M
  *   conv_w  [channels, 4]
  *   out     [total_tokens, channels] = bf16(silu(sum_j x(t-3+j) w[c, j])),
  *           fp32 taps in the order of the decode prologue (yh_gdn_decode_prep)
- * dtype: bf16, alone or | YH_CONV_PLANES(p): out is then p column groups apart,
- * [p, total_tokens, channels / p].
+ * dtype: bf16, alone or | YH_CONV_PLANES(p), p >= 1: out is then p column groups
+ * apart, [p, total_tokens, channels / p].  Any other word is refused.
  */
 #define YH_CONV_PLANES(p) ((p) << 8)
 int yh_conv_prefill(const void* proj, int64_t proj_stride, void* window, const void* conv_w,

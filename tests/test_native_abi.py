@@ -127,3 +127,15 @@ def test_norm_and_reduce_argument_checks(lib):
     assert b"aligned" in lib.yh_last_error()
     assert lib.yh_linear_reduce(fake, ctypes.c_void_p(256 + 2), 2560, 4, 2560, 12, None, 0, None) == -1
     assert lib.yh_linear_reduce(fake, fake, 2560, 4, 2560, 12, ctypes.c_void_p(256 + 4), 2560, None) == -1
+
+
+def test_conv_prefill_dtype_words(lib):
+    """The dtype word holds bf16 and, above it, a number of planes that divides
+    the channels; any other word is refused."""
+    def conv(dtype, channels=48):   # no pieces: nothing is launched
+        return lib.yh_conv_prefill(None, channels, None, None, None, 0, 0, channels, None, dtype, None)
+    assert conv(_native.BF16) == conv(_native.BF16 | 3 << 8) == 0
+    for word in (_native.F16, _native.F32, -255, -1, _native.F16 | 3 << 8, _native.BF16 - (1 << 31)):
+        assert conv(word) == -1 and b"bfloat16" in lib.yh_last_error(), word
+    for planes in (5, 96, 1 << 20):
+        assert conv(_native.BF16 | planes << 8) == -1 and b"divide" in lib.yh_last_error(), planes

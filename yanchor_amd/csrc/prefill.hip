@@ -438,9 +438,8 @@ extern "C" int yh_conv_prefill(const void* proj, int64_t proj_stride, void* wind
   using namespace yh;
   YH_CHECK_ARG(n_seqs >= 0 && total_tokens >= 0 && channels > 0 && proj_stride >= channels,
                "conv_prefill: bad sizes");
+  YH_CHECK_ARG(dtype >= 0 && (dtype & 0xff) == YH_BF16, "conv_prefill: activations must be bfloat16");
   const int64_t planes = dtype >> 8 > 0 ? dtype >> 8 : 1;
-  dtype &= 0xff;
-  YH_CHECK_ARG(dtype == YH_BF16, "conv_prefill: activations must be bfloat16");
   YH_CHECK_ARG(channels % planes == 0, "conv_prefill: planes must divide the channels");
   if (n_seqs == 0) return YH_OK;
   YH_CHECK_ARG(proj && window && conv_w && cu_seqlens && (out || total_tokens == 0), "conv_prefill: null pointer");
