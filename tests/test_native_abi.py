@@ -139,3 +139,17 @@ def test_conv_prefill_dtype_words(lib):
         assert conv(word) == -1 and b"bfloat16" in lib.yh_last_error(), word
     for planes in (5, 96, 1 << 20):
         assert conv(_native.BF16 | planes << 8) == -1 and b"divide" in lib.yh_last_error(), planes
+
+
+@pytest.mark.parametrize("version", [106, 107])
+def test_an_older_library_asks_for_a_rebuild(tmp_path, monkeypatch, version):
+    """A library of the ABI before the anchor-memory token calls, or one that
+    lacks an entry point of its version, is refused with the way out."""
+    import subprocess
+    src, so = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text(f'int yh_abi_version(void) {{ return {version}; }}\nconst char* yh_last_error(void) {{ return ""; }}\n')
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    monkeypatch.setattr(_native, "LIB_PATH", so)
+    monkeypatch.setattr(_native, "_lib", None)
+    with pytest.raises(RuntimeError, match="yanchor_amd.build"):
+        _native.lib()

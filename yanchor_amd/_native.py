@@ -14,8 +14,9 @@ import torch
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libyanchor_amd.so"
 # yh_abi_version() of the library these signatures describe (103: yh_rmsnorm_partials takes
 # out2_stride; 104: yh_linear_pack lays K blocks outermost; 105: yh_rmsnorm_partials takes part2;
-# 106: yh_gdn_decode_fused takes the state dtype)
-ABI_VERSION = 106
+# 106: yh_gdn_decode_fused takes the state dtype; 107: the yh_anchor_tokens_* calls are added,
+# yh_gdn_chunk_varlen uses its workspace, yh_conv_prefill's dtype may hold a number of planes)
+ABI_VERSION = 107
 
 F32, BF16, F16, I32, I64, U8 = 0, 1, 2, 3, 4, 5
 DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16,
@@ -126,12 +127,12 @@ def lib() -> ctypes.CDLL:
         if found != ABI_VERSION:
             raise RuntimeError(f"yanchor_amd native library at {LIB_PATH} has ABI version {found}, these bindings "
                                f"expect {ABI_VERSION}; rebuild it with `python -m yanchor_amd.build`")
-        for name, args in SIGNATURES.items():
-            fn = getattr(handle, name)
-            fn.restype = ctypes.c_int
-            fn.argtypes = args
-        for name, (res, args) in PLAIN.items():
-            fn = getattr(handle, name)
+        entries = {name: (ctypes.c_int, args) for name, args in SIGNATURES.items()}
+        for name, (res, args) in {**entries, **PLAIN}.items():
+            fn = getattr(handle, name, None)
+            if fn is None:
+                raise RuntimeError(f"yanchor_amd native library at {LIB_PATH} has no {name}; rebuild it with "
+                                   "`python -m yanchor_amd.build`")
             fn.restype = res
             fn.argtypes = args
         _lib = handle
