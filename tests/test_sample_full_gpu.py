@@ -57,3 +57,28 @@ def test_full_draws(gpu, v, k, p, ties):
                 for s2 in (-1e-6, 0.0, 1e-6):
                     near.add(_select(kept, mass, max(1, int((u[r] + s2) * cut)))[0])
         assert got[r] in near, (r, got[r], near)
+
+
+@pytest.mark.parametrize("v", [90, 600, 5000])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k,p", [(0, 1.0), (0, 0.9), (80, 0.7)])
+def test_rows_without_probabilities(gpu, v, dtype, k, p):
+    """A NaN, +infinity or nothing above -infinity leaves no mass to draw from:
+    the first element of the order, among rows that draw as they would alone."""
+    gen = torch.Generator().manual_seed(v)
+    x = torch.randn(6, v, generator=gen).to(dtype)
+    x[1, [v // 2, v // 2 + 3]] = float("nan")
+    x[2, [v - 1, 40]] = float("inf")
+    x[3] = float("-inf")
+    x[4, 5:] = float("-inf")          # five finite scores
+    x = x.to(gpu)
+    ids, steps = torch.arange(6, device=gpu) * 5, torch.arange(6, device=gpu)
+
+    def draw(rows):
+        return ik.topk_sample(x[rows], ids[rows], steps[rows], seed=3, temperature=0.8, top_k=k, top_p=p,
+                              mode=ik.SAMPLE_TORCH).flatten().tolist()
+    got = draw(list(range(6)))
+    in_order = k <= 0 and p == 1.0
+    assert got[1:4] == ([0, 0, 0] if in_order else [v // 2, 40, 0])
+    assert 0 <= got[4] < 5
+    assert [got[0], got[4], got[5]] == draw([0]) + draw([4]) + draw([5])

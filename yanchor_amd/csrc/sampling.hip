@@ -708,6 +708,11 @@ namespace {
 // summation order.  The two draws of the value order (the top_p cut and the
 // token) share the first digit's buckets.
 //
+// A row whose S is not a number (a NaN or +infinity among the candidates, or
+// nothing above -infinity) has no mass and draws the first element of the order:
+// index 0 in vocabulary order, the largest score (NaN above all numbers, below
+// them with its sign set; the lower index first) in value order.
+//
 // Bound by the exponentials and the fixed-point conversions of a row on one CU
 // (a third of the time each for S and the first digit).  4-bit digits in
 // registers (13 passes a draw, 16 conditional 64-bit additions an element) took
@@ -801,7 +806,8 @@ __device__ __forceinline__ uint64_t full_key(const FullArgs& a, float x, int i) 
 
 __device__ __forceinline__ uint64_t full_mass(const FullArgs& a, const FullRow& r, float x) {
   const float xt = x / a.temperature;
-  return static_cast<uint64_t>(static_cast<double>(expf(xt - r.mt)) * r.scale);
+  // fmax: no mass where the product is not a number (S is not)
+  return static_cast<uint64_t>(fmax(static_cast<double>(expf(xt - r.mt)) * r.scale, 0.0));
 }
 
 // The buckets of the digit of `width` bits at `pos` of the candidates whose
