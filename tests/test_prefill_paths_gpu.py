@@ -333,6 +333,7 @@ def test_memory_sequence_packed_offsets(gpu, offsets):
     ([129, 0, 64, 700], 2, 8, 128, False, torch.bfloat16),   # an empty sequence, slots between chunks, GQA
     ([500, 1], 3, 27, 128, True, torch.float32),     # two tiles a workgroup
     ([191, 257], 16, 32, 64, True, torch.float32),   # 64 value columns
+    ([300, 200, 257], 8, 32, 64, True, torch.float32),   # two tiles of them a workgroup
 ])
 def test_gdn_few_sequences(gpu, lengths, h, hv, v, h0, gates):
     """The same operations in the same order as the one-launch form: the same
