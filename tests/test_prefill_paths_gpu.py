@@ -277,6 +277,67 @@ def test_memory_sequence_segments(gpu, cap, chunk, length, heads, groups, odd):
     assert torch.equal(again, got[valid.to(gpu)])
 
 
+@pytest.mark.parametrize("cap,chunk,length,heads,groups", [(16, 8, 40, 4, 2), (256, 64, 300, 32, 8), (130, 5, 33, 3, 1)])
+def test_assembled_sequence_calls(gpu, cap, chunk, length, heads, groups):
+    """The C calls that take assembled sources [slots | pending | new tokens] --
+    yh_anchor_prefix, yh_anchor_sequence_read, yh_anchor_sequence_commit -- leave
+    the oracle's state and read, as the calls on tokens in place do."""
+    gen = torch.Generator().manual_seed(cap)
+    b, dt, counts = 3, torch.bfloat16, [length, length // 3, 1]
+    st = _memory_state(gen, b, groups, cap, chunk, [0, chunk - 1, chunk // 2], 2 * cap, dt, True)
+    q, k, v = (torch.randn(b, length, h, 128, generator=gen).to(dt) for h in (heads, groups, groups))
+    sc = torch.randn(b, length, groups, generator=gen)
+    valid = torch.arange(length)[None] < torch.tensor(counts)[:, None]
+    want_state = oracle_memory.MemoryState(**{f.name: getattr(st, f.name).clone() for f in fields(st)})
+    want = oracle_memory.sequence(q, k, v, sc, valid, chunk, want_state)
+    src = [torch.cat((c.transpose(1, 2), p[:, :, :chunk].transpose(1, 2), x), 1).contiguous().to(gpu)
+           for c, p, x in ((st.keys, st.pending_keys, k), (st.values, st.pending_values, v))]
+    got = _clone(st, gpu)
+    q, sc, n = q.to(gpu), sc.to(gpu), torch.tensor(counts, device=gpu)
+    blocks, total = -(-length // chunk) + 1, cap + chunk + length
+    block_refs = torch.empty(b, blocks, groups, cap, dtype=torch.int32, device=gpu)
+    final, pending = torch.empty_like(block_refs[:, 0]), torch.empty(b, groups, chunk, dtype=torch.int32, device=gpu)
+    out, stream = torch.empty_like(q), _native.stream_of(q)
+    _native.call("yh_anchor_prefix", sc.data_ptr(), n.data_ptr(), got.scores.data_ptr(), got.positions.data_ptr(),
+                 got.pending_scores.data_ptr(), got.count.data_ptr(), got.total.data_ptr(), block_refs.data_ptr(),
+                 final.data_ptr(), pending.data_ptr(), b, length, groups, cap, chunk, chunk, blocks, stream)
+    _native.call("yh_anchor_sequence_read", q.data_ptr(), src[0].data_ptr(), src[1].data_ptr(), block_refs.data_ptr(),
+                 _native.I32, got.count.data_ptr(), out.data_ptr(), b, length, blocks, chunk, heads, groups, 128, total,
+                 cap, _native.BF16, stream)
+    _native.call("yh_anchor_sequence_commit", src[0].data_ptr(), src[1].data_ptr(), final.data_ptr(),
+                 pending.data_ptr(), n.data_ptr(), got.keys.data_ptr(), got.values.data_ptr(),
+                 got.pending_keys.data_ptr(), got.pending_values.data_ptr(), got.count.data_ptr(),
+                 got.total.data_ptr(), b, total, length, groups, cap, chunk, chunk, 128, _native.BF16, stream)
+    for f in fields(st):
+        assert torch.equal(getattr(got, f.name).cpu().double(), getattr(want_state, f.name).double()), f.name
+    diff = (out.cpu().double() - want.double())[valid]
+    assert diff.norm() <= 1e-2 * want.double()[valid].norm()
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 128), (torch.float32, 20)])
+@pytest.mark.parametrize("cap,pc,chunk", [(4090, 20, 16), (4096, 4200, 7), (4095, 1, 1), (31, 70, 64)])
+def test_commit_from_other_sources(gpu, cap, pc, chunk, dtype, d):
+    """Rows past one stage of the commit (4096), exactly: every slot takes the
+    source row it names, or zeros; the counters advance."""
+    gen = torch.Generator().manual_seed(cap + pc)
+    b, g, s, length = 2, 3, 500, 9
+    src = torch.randn(2, b, s, g, d, generator=gen).to(dtype)
+    refs = [torch.randint(-40, s + 40, (b, g, n), generator=gen).to(torch.int32) for n in (cap, pc)]
+    rows, counts = torch.full((2, b, g, cap, d), 7.0).to(dtype), torch.tensor([length, 4])
+    pend, count, total = torch.full((2, b, g, pc, d), 7.0).to(dtype), torch.tensor([chunk - 1, 0]), torch.tensor([90, 80])
+
+    def take(which, ref):
+        at = ref.clamp(0, s - 1).long()
+        x = src[which][torch.arange(b)[:, None, None], at, torch.arange(g)[None, :, None]]
+        return x.masked_fill(((ref < 0) | (ref >= s))[..., None], 0)
+    dev = [x.to(gpu) for x in (src[0], src[1], *refs, counts, rows[0], rows[1], pend[0], pend[1], count, total)]
+    _native.call("yh_anchor_sequence_commit", *[x.data_ptr() for x in dev], b, s, length, g, cap, pc, chunk, d,
+                 _native.code(src), _native.stream_of(dev[0]))
+    for x, want in zip(dev[5:9], (take(0, refs[0]), take(1, refs[0]), take(0, refs[1]), take(1, refs[1]))):
+        assert torch.equal(x.cpu(), want)
+    assert torch.equal(dev[9].cpu(), (count + counts) % chunk) and torch.equal(dev[10].cpu(), total + counts)
+
+
 @pytest.mark.parametrize("case", ["float32", "heads of 64", "5 heads on 2 groups", "no tokens", "unaligned keys"])
 @pytest.mark.parametrize("packed", [False, True])
 def test_memory_sequence_refusals_leave_the_state(gpu, case, packed):
