@@ -314,6 +314,28 @@ def test_assembled_sequence_calls(gpu, cap, chunk, length, heads, groups):
     assert diff.norm() <= 1e-2 * want.double()[valid].norm()
 
 
+def test_prefix_past_a_grid_row(gpu):
+    """More memories than one grid row of its workgroups holds threads for: one
+    slot and one token each, the better of the two stays."""
+    b, g = (1 << 22) // 8 + 3, 8
+    score, pos = torch.randn(b, g, 1, device=gpu), torch.zeros(b, g, 1, dtype=torch.int32, device=gpu)
+    new, old = torch.randn(b, 1, g, device=gpu), score.clone()
+    pend, count, total = torch.zeros(b, g, 1, device=gpu), torch.zeros(b, dtype=torch.long, device=gpu), \
+        torch.full((b,), 5, dtype=torch.long, device=gpu)
+    ones = torch.ones_like(count)
+    refs = torch.full((3, b, g, 1), -7, dtype=torch.int32, device=gpu)     # of the block, final, pending
+    _native.call("yh_anchor_prefix", new.data_ptr(), ones.data_ptr(), score.data_ptr(), pos.data_ptr(), pend.data_ptr(),
+                 count.data_ptr(), total.data_ptr(), refs[0].data_ptr(), refs[1].data_ptr(), refs[2].data_ptr(), b, 1,
+                 g, 1, 1, 1, 1, _native.stream_of(new))
+    fresh = new.transpose(1, 2)
+    kept = (fresh > old)
+    sure = fresh != old
+    assert torch.equal(score, torch.maximum(fresh, old))
+    assert torch.equal(pos[sure], (kept * 5).to(torch.int32)[sure])
+    assert not refs[0].any() and torch.equal(refs[1][sure], (kept * 2).to(torch.int32)[sure])
+    assert (refs[2] == -1).all() and torch.isinf(pend).all()
+
+
 @pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 128), (torch.float32, 20)])
 @pytest.mark.parametrize("cap,pc,chunk", [(4090, 20, 16), (4096, 4200, 7), (4095, 1, 1), (31, 70, 64)])
 def test_commit_from_other_sources(gpu, cap, pc, chunk, dtype, d):

@@ -58,6 +58,7 @@ struct PrefixArgs {
   int32_t* final_refs;      // [B, G, KC]
   int32_t* pending_refs;    // [B, G, PC]
   int L, G, KC, PC, C, NB;
+  int64_t groups;           // B * G
 };
 
 // Sort the n candidates key[0][0, n) (and idx[0]) into rank order: runs of
@@ -138,7 +139,8 @@ __global__ void __launch_bounds__(kSortThreads) anchor_prefix_kernel(PrefixArgs 
   __shared__ float opend[kSeqMaxChunk];
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int64_t bg = blockIdx.x;
+  const int64_t bg = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
+  if (bg >= a.groups) return;
   const int64_t b = bg / a.G;
   const int g = static_cast<int>(bg % a.G);
   const int KC = a.KC, C = a.C, G = a.G;
@@ -332,7 +334,7 @@ int launch_prefix(PrefixArgs a, int64_t B, int64_t L, int64_t G, int64_t capacit
   YH_CHECK_ARG(capacity + chunk <= kSeqMaxCand, "%s: capacity + chunk must be <= %d", what, kSeqMaxCand);
   YH_CHECK_ARG(NB * chunk >= L + chunk - 1, "%s: %lld blocks of %lld cannot hold %lld pending + new tokens", what,
                (long long)NB, (long long)chunk, (long long)(L + chunk - 1));
-  YH_CHECK_ARG(capacity + chunk + L < (1LL << 31) && B * G < (1LL << 32) / kSortThreads, "%s: too large", what);
+  YH_CHECK_ARG(capacity + chunk + L < (1LL << 31) && B * G < (1LL << 31), "%s: too large", what);
   if (B == 0) return YH_OK;
   YH_CHECK_ARG(a.counts && a.scores && a.pos && a.pscores && a.count && a.total && a.final_refs && a.pending_refs &&
                    (L == 0 || a.new_scores) && (NB == 0 || a.block_refs),
@@ -343,8 +345,10 @@ int launch_prefix(PrefixArgs a, int64_t B, int64_t L, int64_t G, int64_t capacit
   a.PC = static_cast<int>(pending_capacity);
   a.C = static_cast<int>(chunk);
   a.NB = static_cast<int>(NB);
-  hipLaunchKernelGGL(anchor_prefix_kernel, dim3(static_cast<unsigned>(B * G)), dim3(kSortThreads), 0,
-                     static_cast<hipStream_t>(stream), a);
+  a.groups = B * G;
+  const int64_t wide = a.groups < (1 << 20) ? a.groups : 1 << 20;   // a grid's row holds less than 2^32 threads
+  const dim3 grid(static_cast<unsigned>(wide), static_cast<unsigned>((a.groups + wide - 1) / wide));
+  hipLaunchKernelGGL(anchor_prefix_kernel, grid, dim3(kSortThreads), 0, static_cast<hipStream_t>(stream), a);
   YH_CHECK_LAUNCH(what);
   return YH_OK;
 }
