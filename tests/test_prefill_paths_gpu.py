@@ -123,6 +123,23 @@ def test_swa_prefill_unseen_values(gpu, heads, groups, tt, bad):
         assert torch.equal(got[last:], clean[last:]), at
 
 
+def test_swa_prefill_past_a_grid_row(gpu):
+    """More tiles than one grid row holds threads for: the first of two pieces
+    over and over, then the second once."""
+    n, g, bf = 3, 8, torch.bfloat16
+    q, k, v = (torch.randn(n, g, 128, device=gpu).to(bf) for _ in range(3))
+    ring, at = torch.zeros(2, g, 64, 128, dtype=bf, device=gpu), torch.zeros(2, dtype=torch.long, device=gpu)
+    rows, cu = torch.arange(2, device=gpu), _cu([1, 2], gpu)
+    want = layers.swa_prefill(q, k, v, cu, at, ring, ring, rows)
+    tiles = torch.zeros((1 << 22) + 5, 2, dtype=torch.int32, device=gpu)
+    tiles[-1, 0] = 1
+    out = torch.full_like(q, 7.0)
+    _native.call("yh_swa_prefill", q.data_ptr(), g * 128, k.data_ptr(), g * 128, v.data_ptr(), g * 128,
+                 ring.data_ptr(), ring.data_ptr(), rows.data_ptr(), at.data_ptr(), cu.data_ptr(), tiles.data_ptr(),
+                 len(tiles), None, 0, 0, out.data_ptr(), 2, 2, g, g, 128, 64, _native.BF16, _native.stream_of(q))
+    assert torch.equal(out, want)
+
+
 def test_swa_prefill_scattered_tiles(gpu):
     """A caller's tile list whose neighbours lie far apart costs about what the
     sorted list does (each tile its own window, at most twice the copies): the

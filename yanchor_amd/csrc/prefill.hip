@@ -232,7 +232,8 @@ struct SwaArgs {
 
 // Workgroup id: the KV group is the fastest index, so with 8 groups every XCD
 // keeps one group's keys and values in its L2 while neighbouring tiles, whose
-// windows overlap by all but a tile, run on it.
+// windows overlap by all but a tile, run on it.  (A grid's row holds less than
+// 2^32 threads: longer lists take further rows.)
 template <int DT, int NW>
 __global__ void __launch_bounds__(NW * 64, 2) swa_prefill_kernel(SwaArgs a) {
   using M = attn::Mfma<DT>;
@@ -242,7 +243,8 @@ __global__ void __launch_bounds__(NW * 64, 2) swa_prefill_kernel(SwaArgs a) {
 
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = blockIdx.x % a.G;
-  const int64_t first = static_cast<int64_t>(blockIdx.x / a.G) * kTiles;
+  const int64_t first = (static_cast<int64_t>(blockIdx.y) * (gridDim.x / a.G) + blockIdx.x / a.G) * kTiles;
+  if (first >= a.n_tiles) return;
   const int count = static_cast<int>(a.n_tiles - first < kTiles ? a.n_tiles - first : kTiles);
   const int32_t* list = a.tiles + 2 * first;
   const int R = a.H / a.G, TT = attn::kTile / R, W = a.W;
@@ -500,8 +502,7 @@ extern "C" int yh_swa_prefill(const void* q, int64_t q_stride, const void* k, in
                "swa_prefill: token strides must hold whole heads and keep 16-byte rows");
   YH_CHECK_ARG(!gate || (gate_head_stride >= D && gate_token_stride >= H * gate_head_stride),
                "swa_prefill: bad gate strides");
-  YH_CHECK_ARG(n_tiles < (1ll << 32) / (G * 128) && G < 65536 && window < (1ll << 30),
-               "swa_prefill: grid too large");
+  YH_CHECK_ARG(n_tiles < (1ll << 31) && G < 65536 && window < (1ll << 30), "swa_prefill: grid too large");
   const bool off32 = k_stride < (1ll << 23) && v_stride < (1ll << 23) && window < (1ll << 22);
   const bool gate16 = gate && aligned16(gate) && gate_token_stride % 8 == 0 && gate_head_stride % 8 == 0;
   SwaArgs a{static_cast<const uint16_t*>(q), q_stride, static_cast<const uint16_t*>(k), k_stride,
@@ -513,7 +514,9 @@ extern "C" int yh_swa_prefill(const void* q, int64_t q_stride, const void* k, in
   // prompts (385 and 390 us at 16 pieces of 15,465 tokens with context) and
   // short ones leave the chip emptier (45 and 38 us for 1000 tokens).
   constexpr int kWaves = 4;
-  const dim3 grid(static_cast<unsigned>((n_tiles + kWaves / 2 - 1) / (kWaves / 2) * G)), block(kWaves * 64);
+  const int64_t pairs = (n_tiles + kWaves / 2 - 1) / (kWaves / 2), row = ((1ll << 32) / (kWaves * 64) - 1) / G;
+  const int64_t wide = pairs < row ? pairs : row;
+  const dim3 grid(static_cast<unsigned>(wide * G), static_cast<unsigned>((pairs + wide - 1) / wide)), block(kWaves * 64);
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == YH_BF16)
     hipLaunchKernelGGL((swa_prefill_kernel<YH_BF16, kWaves>), grid, block, 0, st, a);
