@@ -13,20 +13,21 @@
 //
 // What bounds it: the softmax's vector work (a fma, a quarter-rate exp2, half a
 // conversion and an addition a score, and a rescaling of the accumulators a
-// tile) and the MFMAs take 1300 and 1024 cycles of a SIMD a
-// tile; two waves a SIMD overlap them only in part, the rest is waits on LDS
-// and on the tile's barrier.  Hence: key tiles by direct global-to-LDS copies,
-// double buffered, one barrier a tile; 16-byte pieces swizzled so that the
-// 16-byte K reads and the transposing V reads hit distinct banks; a few
-// operands read ahead of their MFMA; the exponentials of one step of the value
-// product between the MFMAs of the step before; a raised wave priority around
-// the MFMAs, so that they run under the other wave's vector work; no mask code on
-// tiles where every key is live.  Six waves a workgroup (three a SIMD, 168
-// registers) take 1.4 times as long even with the addresses re-formed a tile.  The
-// denominator sums P in float32, before the rounding that the value product
-// sees.  (A running maximum that lags the scores by up to 2^8 and leaves out most rescalings was
-// 10 % faster and 2 % further from float64: a row's largest probability is
-// exact only while the maximum is.)
+// tile).  A wave's tile costs a SIMD 3460 cycles in window attention over 16
+// pieces of 15,465 tokens with full rings: vector instructions issue in 1970 of
+// them, the MFMAs take 1024, and two waves a SIMD overlap the two only in part;
+// the rest is waits on LDS and on the tile's barrier.  Hence: key tiles by direct
+// global-to-LDS copies, double buffered, one barrier a tile; 16-byte pieces
+// swizzled so that the 16-byte K reads and the transposing V reads hit distinct
+// banks; a few operands read ahead of their MFMA; the exponentials of one step of
+// the value product between the MFMAs of the step before; a raised wave priority
+// around the MFMAs, so that they run under the other wave's vector work; no mask
+// code on tiles where every key is live.  Six waves a workgroup (three a SIMD,
+// 168 registers) take 1.4 times as long even with the addresses re-formed a
+// tile.  The denominator sums P in float32, before the rounding that the value
+// product sees.  (A running maximum that lags the scores by up to 2^8 and leaves
+// out most rescalings was 10 % faster and 2 % further from float64: a row's
+// largest probability is exact only while the maximum is.)
 #pragma once
 #include "common.h"
 
@@ -233,7 +234,8 @@ struct State {
       ph[ks & 1][e] = h;
       den += p0 + p1;
       if constexpr (HILO)
-        pl[ks & 1][e] = M::round2(p0 - M::widen(static_cast<uint16_t>(h)), p1 - M::widen(static_cast<uint16_t>(h >> 16)));
+        pl[ks & 1][e] =
+            M::round2(p0 - M::widen(static_cast<uint16_t>(h)), p1 - M::widen(static_cast<uint16_t>(h >> 16)));
     };
     // word e of a V operand of step ks holds keys 16 ks + 8 (e / 2) + 4 half + 2 (e % 2) and the next
     uint32_t kept[4];

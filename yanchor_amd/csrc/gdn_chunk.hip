@@ -12,14 +12,14 @@
 //
 // T and A = Q K^T o Gamma do not depend on the state S.  chunk_fused_kernel
 // runs one workgroup per (sequence, value head) that walks the sequence's chunks
-// (few sequences: chunk_prep_kernel and chunk_scan_kernel below).  Eight scan waves hold the 128 x V fp32 state in MFMA
-// accumulators (wave w owns value columns 16w..16w+15) and run the
-// state-dependent products of chunk j - 1 (Q S and K S, v_new, o, the state
-// update, with S and v_new never leaving registers) while four prep waves
-// (with help from the scan waves where those have time to spare) prepare chunk
-// j: decays, K K^T and Q K^T with the L2 norms from their diagonals, the fp32
-// inverse T on MFMA block products, A, the scalings.  Only q, k, v, the gates,
-// o and the states cross HBM.
+// (few sequences: chunk_prep_kernel and chunk_scan_kernel below).  Eight scan
+// waves hold the 128 x V fp32 state in MFMA accumulators (wave w owns value
+// columns 16w..16w+15) and run the state-dependent products of chunk j - 1 (Q S
+// and K S, v_new, o, the state update, with S and v_new never leaving registers)
+// while four prep waves (with help from the scan waves where those have time to
+// spare) prepare chunk j: decays, K K^T and Q K^T with the L2 norms from their
+// diagonals, the fp32 inverse T on MFMA block products, A, the scalings.  Only q,
+// k, v, the gates, o and the states cross HBM.
 // Per-token L2 norms, beta and decays are diagonal factors, so products with
 // the raw q / k / v tensors take exact bf16 MFMA operands and the factors go
 // into the epilogues or the fp32 operand.  Products whose operands are fp32 on
@@ -1129,8 +1129,10 @@ __global__ void __launch_bounds__(CT * 256) chunk_scan_kernel(FusedArgs a, const
 
 // The split form pays while its scan, 4 workgroups a head of 128 columns, runs
 // in one round (one workgroup a CU) and a sequence has a few chunks on average.
-// Two sequences x 32 heads: 113 us against 165; four of 4000 tokens: 417 against
-// 361.  One sequence of 300 tokens: 32 against 46; of 50: 43 against 40.
+// us of both launches against the one, 32 heads: a sequence of 3001 tokens 109
+// and 241, of 300 19 and 31, of 100 13 and 16, of 50 12 and 10.5; two of 1000 and
+// 2000 90 and 166; four of 4000 356 and 328, of 1000 100 and 88.  (128 tokens lie
+// on the safe side of the crossing.)
 bool split_form(int64_t total_tokens, int64_t n_seqs, int64_t HV, int64_t V) {
   return n_seqs * HV * (V / 32) <= 256 && total_tokens > 128 * n_seqs &&
          (total_tokens / kC + n_seqs) * HV * kRecord * 16 <= (1LL << 31);   // scratch of at most 2 GiB
@@ -1183,8 +1185,8 @@ extern "C" int yh_gdn_chunk_varlen(const void* q, const void* k, const void* v, 
     uint4* ws = static_cast<uint4*>(workspace);
     hipLaunchKernelGGL(chunk_prep_kernel, dim3(static_cast<unsigned>(slots * HV)), dim3(256), 0, st, f, ws);
     YH_CHECK_LAUNCH("gdn_chunk prep");
-    // one tile a workgroup where that still is one round (151 against 161 us for
-    // one sequence of 3001 tokens x 32 heads)
+    // one tile a workgroup where that still is one round (both launches 109 us
+    // against 117 with two, one sequence of 3001 tokens x 32 heads)
     const bool one = n_seqs * HV * (V / 16) <= 256;
     if (V == 128 && one) launch_scan<128, 1>(f, ws, st);
     else if (V == 128) launch_scan<128, 2>(f, ws, st);

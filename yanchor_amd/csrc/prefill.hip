@@ -24,8 +24,8 @@
 //
 // swa_prefill_kernel: a tile is 64 query rows, 64 / R consecutive tokens x the
 // R query heads of a KV group.  A workgroup of NW waves takes NW / 2 tiles that
-// follow each other in the list, two waves each; the tiles of one piece share
-// their key tiles (attn_tile.h).
+// follow each other in the list, two waves each; tiles of one piece whose windows
+// meet share their key tiles (attn_tile.h).
 #include <type_traits>
 
 #include "attn_tile.h"
@@ -89,15 +89,15 @@ struct Chan<1> {
 
 constexpr int kConvBatch = 4;  // rows in flight per thread
 
-// Bound by HBM (each input row read once, each output row written once) with
-// the SiLU's exact exp and division close behind on the VALU.  A thread owns
-// VEC channels and walks a run of `run` tokens with the three earlier inputs
-// and the four taps in registers, so a row is loaded once (plus three halo
-// rows a run) in 16-byte accesses, four rows ahead of their use.  One token
-// and one channel a thread (2-byte accesses, every row loaded four times, a
-// sequence search a workgroup) took 976 us at 64 pieces of 17,400 tokens x
-// 12288 channels (871 MB); this takes 247 us with the
-// host's checks.
+// Bound by the VALU, which issues in 86 % of the cycles: 35 issue slots an
+// element, most of them the SiLU's exact exp and division (HBM would take 140 us
+// of the 240 below).  A thread owns VEC channels and walks a run of `run` tokens
+// with the three earlier inputs and the four taps in registers, so a row is
+// loaded once (plus three halo rows a run) in 16-byte accesses, four rows ahead
+// of their use.  One token and one channel a thread (2-byte accesses, every row
+// loaded four times, a sequence search a workgroup) took 976 us at 64 pieces of
+// 17,400 tokens x 12288 channels (871 MB); this takes 247 us with the host's
+// checks.
 template <int VEC>
 __global__ void __launch_bounds__(256) conv_prefill_kernel(ConvArgs a, int64_t total, int run) {
   using Ch = Chan<VEC>;
@@ -516,7 +516,8 @@ extern "C" int yh_swa_prefill(const void* q, int64_t q_stride, const void* k, in
   constexpr int kWaves = 4;
   const int64_t pairs = (n_tiles + kWaves / 2 - 1) / (kWaves / 2), row = ((1ll << 32) / (kWaves * 64) - 1) / G;
   const int64_t wide = pairs < row ? pairs : row;
-  const dim3 grid(static_cast<unsigned>(wide * G), static_cast<unsigned>((pairs + wide - 1) / wide)), block(kWaves * 64);
+  const dim3 grid(static_cast<unsigned>(wide * G), static_cast<unsigned>((pairs + wide - 1) / wide));
+  const dim3 block(kWaves * 64);
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == YH_BF16)
     hipLaunchKernelGGL((swa_prefill_kernel<YH_BF16, kWaves>), grid, block, 0, st, a);

@@ -716,8 +716,9 @@ namespace {
 // Bound by the exponentials and the fixed-point conversions of a row on one CU
 // (a third of the time each for S and the first digit).  4-bit digits in
 // registers (13 passes a draw, 16 conditional 64-bit additions an element) took
-// 2259 us at 30 rows x 151936 bf16, top_p 0.95; this takes 418 us (top_p 1, in
-// vocabulary order: 574 and 254; 160 rows: 3293 and 558).
+// 2175 us at 30 rows x 151936 bf16 with the presence penalty, top_p 0.95; this
+// takes 395 us (top_p 1, in vocabulary order: 569 and 249; 160 rows: 3180 and
+// 517).
 constexpr int kFullThreads = 1024;
 constexpr int kFullWaves = kFullThreads / kWave;
 constexpr int kFullDigit = 12;
