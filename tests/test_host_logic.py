@@ -5,6 +5,7 @@
 * ``_should_compact_dynamic_decode_tail`` (1348-1349): the boundary cases;
 * ``synthetic_requests``: the backlog that fills the batch arrives at step 0.
 """
+import pytest
 import torch
 
 from yanchor_amd import inference_kernels as ik
@@ -102,3 +103,34 @@ def test_text_ids_round_trip():
     assert all(0 <= i < 256 for i in ids)
     assert inference.decode_ids(ids) == "héllo, world"
     assert inference.decode_ids([104, 105, 5000]) == "hi�"
+
+
+def test_prefill_checks_of_many_pieces():
+    """The host's checks of a packed prefill do no Python work a piece (60 to
+    100 ms at a million pieces when they did, a few ms in tensor operations), and
+    refuse what they refused."""
+    import time
+    from yanchor_amd import layers
+    r = 1 << 20
+    cu, starts, rows = torch.arange(r + 1, dtype=torch.int32), torch.zeros(r, dtype=torch.long), torch.arange(r) % 8
+    times = []
+    for _ in range(5):
+        t = time.perf_counter()
+        got, offsets, st, rr = layers._cu(cu, "cpu", r, starts, rows, 8)
+        times.append(time.perf_counter() - t)
+    assert min(times) < 0.03, times
+    assert torch.equal(torch.as_tensor(offsets), cu.long()) and torch.equal(rr, rows) and torch.equal(st, starts)
+    for rep in (1, 50):   # both sides of the line between lists and tensors
+        n = 5 * rep
+        base = [0] + [x + 5 * i for i in range(rep) for x in (2, 2, 5)]
+        ok = (torch.tensor(base), "cpu", n, torch.tensor([0, 3, 9] * rep), torch.tensor([-1, 1, 0] * rep), 2)
+        assert list(layers._cu(*ok)[1]) == base
+        for at, bad in ((0, [1, *base[1:]]), (0, [0, 3, *base[2:]]), (0, [*base[:-1], n + 1]), (3, [0, -1, 9] * rep),
+                        (4, [0, 1, 2] * rep), (3, [0, 3, 9] * rep + [1]), (4, [0, 1, 0] * rep + [0])):
+            args = list(ok)
+            args[at] = torch.tensor(bad)
+            with pytest.raises(ValueError):
+                layers._cu(*args)
+    assert layers.prefill_tiles([3, 0, 5], 4, "cpu").tolist() == [[0, 0], [2, 0], [2, 4]]
+    assert layers.prefill_tiles(torch.tensor([3, 0, 5]), 4, "cpu").tolist() == [[0, 0], [2, 0], [2, 4]]
+    assert layers.prefill_tiles([], 4, "cpu").shape == (0, 2)

@@ -468,25 +468,31 @@ def _cu(cu_seqlens, device, total, starts=None, ring_rows=None, ring_batch=0):
     so a copy to the host is possible, but it waits for the stream: everything
     that is checked comes in one.  The small per-piece vectors may come from
     the host; the activations and caches must be device tensors.  Returns (cu,
-    its values on the host, starts, ring_rows)."""
+    its values on the host -- a list, or a tensor where they are many --, starts,
+    ring_rows)."""
     cu = cu_seqlens.to(device=device, dtype=torch.int32).contiguous()
     if cu.ndim != 1 or cu.numel() < 1:
         raise ValueError("cu_seqlens must be a 1-D offset vector")
     m, st, rr = cu.numel(), None, None
     if starts is None:
-        h = cu.tolist()
+        h = cu.cpu()
     else:
         st = starts.to(device=device, dtype=torch.int64).contiguous()
         rr = ring_rows.to(device=device, dtype=torch.int64).contiguous()
-        h = torch.cat((cu, st.reshape(-1), rr.reshape(-1))).tolist()
-    if h[0] != 0 or h[m - 1] > total or any(h[i + 1] < h[i] for i in range(m - 1)):
+        h = torch.cat((cu, st.reshape(-1), rr.reshape(-1))).cpu()
+    many = m > 128   # Python takes 0.1 us a piece, tensor operations 8 us a call
+    h = h if many else h.tolist()
+    off = h[:m]
+    falls = bool((off[1:] < off[:-1]).any()) if many else any(b < a for a, b in zip(off, off[1:]))
+    if off[0] != 0 or off[-1] > total or falls:
         raise ValueError("cu_seqlens must be non-decreasing offsets from 0 within the packed tokens")
     if starts is not None:
         if st.shape != (m - 1,) or rr.shape != (m - 1,):
             raise ValueError("starts / ring_rows must hold one entry per piece")
-        if m > 1 and (min(h[m: 2 * m - 1]) < 0 or max(h[2 * m - 1:]) >= ring_batch):
+        first, rows = h[m: 2 * m - 1], h[2 * m - 1:]
+        if m > 1 and ((first.min() if many else min(first)) < 0 or (rows.max() if many else max(rows)) >= ring_batch):
             raise ValueError("starts must be >= 0 and ring rows inside the ring")
-    return cu, h[:m], st, rr
+    return cu, off, st, rr
 
 
 def conv_prefill(proj, window, conv_w, cu_seqlens, channels, planes=1):
@@ -509,7 +515,7 @@ def conv_prefill(proj, window, conv_w, cu_seqlens, channels, planes=1):
         raise ValueError("window must be contiguous [R, 3, channels]")
     if conv_w.shape != (channels, 4) or not conv_w.is_contiguous():
         raise ValueError("conv_w must be contiguous [channels, 4]")
-    if offsets[-1] != n:
+    if int(offsets[-1]) != n:
         raise ValueError("cu_seqlens must cover every packed token")
     if planes < 1 or channels % planes:
         raise ValueError("planes must divide the channels")
@@ -522,10 +528,11 @@ def conv_prefill(proj, window, conv_w, cu_seqlens, channels, planes=1):
 def prefill_tiles(lengths, tokens_per_tile, device):
     """(piece, first token) int32 [n_tiles, 2] of the tiles of
     ``tokens_per_tile`` tokens that cover pieces of the given host lengths."""
-    n = torch.as_tensor([int(x) for x in lengths], dtype=torch.int64)
+    n = lengths.to("cpu", torch.int64) if torch.is_tensor(lengths) else torch.tensor([int(x) for x in lengths],
+                                                                                     dtype=torch.int64, device="cpu")
     count = (n + tokens_per_tile - 1).clamp_min(0) // tokens_per_tile
-    piece = torch.repeat_interleave(torch.arange(n.numel()), count)
-    first = (torch.arange(piece.numel()) - (count.cumsum(0) - count)[piece]) * tokens_per_tile
+    piece = torch.repeat_interleave(torch.arange(n.numel(), device="cpu"), count)
+    first = (torch.arange(piece.numel(), device="cpu") - (count.cumsum(0) - count)[piece]) * tokens_per_tile
     return torch.stack((piece, first), 1).to(torch.int32).to(device)
 
 
@@ -562,11 +569,12 @@ def swa_prefill(q, k, v, cu_seqlens, starts, ring_k, ring_v, ring_rows, *, gate=
     r = cu.numel() - 1
     if 64 % (h // g):
         raise ValueError("query heads per KV head must divide 64")
-    lengths = [b - a for a, b in zip(offsets, offsets[1:])]
+    lengths = [b - a for a, b in zip(offsets, offsets[1:])] if isinstance(offsets, list) else \
+        offsets[1:] - offsets[:-1]
     if tiles is None:
         tiles = prefill_tiles(lengths, 64 // (h // g), dev)
     else:
-        th = tiles.cpu()
+        th, lengths = tiles.cpu(), lengths if isinstance(lengths, list) else lengths.tolist()
         if tiles.dtype != torch.int32 or tiles.ndim != 2 or tiles.shape[1] != 2 or \
                 any(not (0 <= int(p) < r and 0 <= int(t) < lengths[int(p)]) for p, t in th.tolist()):
             raise ValueError("tiles must be int32 (piece, first token) pairs inside the pieces")
